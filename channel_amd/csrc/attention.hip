@@ -697,14 +697,17 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float *__restrict__ ws
 }
 
 // Four consecutive output values at element offset o: fp32 into out, or
-// bf16 into outb when it is set (the operand of the next contraction).
+// bf16 into outb (xb_at order for ntt) when it is set (the operand of the
+// next contraction).
 typedef __bf16 bf16x2a __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void store_out4(float *out, __bf16 *outb, size_t o, f4 v) {
+__device__ __forceinline__ void store_out4(float *out, __bf16 *outb, uint32_t ntt, uint32_t width, uint32_t t,
+                                           uint32_t k, f4 v) {
     if (outb) {
-        *(bf16x2a *)(outb + o) = bf16x2a{(__bf16)v.x, (__bf16)v.y};
-        *(bf16x2a *)(outb + o + 2) = bf16x2a{(__bf16)v.z, (__bf16)v.w};
+        __bf16 *o = outb + xb_at(ntt, width, t, k);
+        *(bf16x2a *)o = bf16x2a{(__bf16)v.x, (__bf16)v.y};
+        *(bf16x2a *)(o + 2) = bf16x2a{(__bf16)v.z, (__bf16)v.w};
     } else {
-        *(f4 *)(out + o) = v;
+        *(f4 *)(out + (size_t)t * width + k) = v;
     }
 }
 
@@ -717,7 +720,7 @@ __global__ __launch_bounds__(256) void k_prefill_attn(const float *__restrict__ 
                                                       const uint32_t *__restrict__ slots, uint32_t num_prev,
                                                       uint32_t num_q_heads, uint32_t kv_dim, float scale,
                                                       uint32_t window, float *__restrict__ out,
-                                                      __bf16 *__restrict__ outb) {
+                                                      __bf16 *__restrict__ outb, uint32_t ntt) {
     constexpr int D = DV * 256;
     const uint32_t t = blockIdx.x, kvh = blockIdx.y;
     const uint32_t S = num_prev + t + 1;
@@ -743,8 +746,7 @@ __global__ __launch_bounds__(256) void k_prefill_attn(const float *__restrict__ 
 #pragma unroll
     for (int h = 0; h < GQA; ++h) inv[h] = 1.0f / (st.l[h] + 1e-9f);
     attn_reduce<DV, GQA>(st, pacc, [&](int h, int col, f4 v) {
-        const size_t o = q_row + (size_t)(kvh * GQA + h) * D + 4 * col;
-        store_out4(out, outb, o, v * inv[h]);
+        store_out4(out, outb, ntt, num_q_heads * D, t, (kvh * GQA + h) * D + 4 * col, v * inv[h]);
     });
 }
 
@@ -905,7 +907,7 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
                                                          uint32_t nfch, uint32_t num_prev, uint32_t n_tok,
                                                          uint32_t num_q_heads, float scale, uint32_t window,
                                                          float *__restrict__ out, __bf16 *__restrict__ outb,
-                                                         float *__restrict__ ws, uint32_t maxparts) {
+                                                         float *__restrict__ ws, uint32_t maxparts, uint32_t ntt) {
     constexpr int D = 256, NK = kPaNK, TQ = 16 * kPaWaves / GQA;
     __shared__ __attribute__((aligned(16))) unsigned char ring[2][kPaChunkBytes];   // two chunks in flight
 
@@ -1108,7 +1110,7 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
     }
     const float inv = 1.0f / (l + 1e-9f);
 #pragma unroll
-    for (int dt = 0; dt < 16; ++dt) store_out4(out, outb, orow + 16 * dt, o[dt] * inv);
+    for (int dt = 0; dt < 16; ++dt) store_out4(out, outb, ntt, num_q_heads * D, tq, head * D + 4 * g + 16 * dt, o[dt] * inv);
 }
 
 // The key-split parts' states of each (token, head) rescaled to their
@@ -1116,7 +1118,8 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
 // that were not split were written by the attention itself.
 __global__ __launch_bounds__(256) void k_prefill_attn_merge(const float *__restrict__ ws, PaGeom geo,
                                                             uint32_t num_q_heads, size_t nrow, uint32_t D,
-                                                            float *__restrict__ out, __bf16 *__restrict__ outb) {
+                                                            float *__restrict__ out, __bf16 *__restrict__ outb,
+                                                            uint32_t ntt) {
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;   // element of [token][head][D]
     if (i >= nrow * D) return;
     const size_t row = i / D;
@@ -1153,7 +1156,8 @@ __global__ __launch_bounds__(256) void k_prefill_attn_merge(const float *__restr
         t += v[p] * a;
         den += lp[p] * a;
     }
-    store_out4(out, outb, i, t * (1.0f / (den + 1e-9f)));
+    const uint32_t width = num_q_heads * D;
+    store_out4(out, outb, ntt, width, (uint32_t)(i / width), (uint32_t)(i % width), t * (1.0f / (den + 1e-9f)));
 }
 
 static int launch_decode_impl(chn_ctx *ctx, const float *q, float *kc, float *vc, const uint32_t *slots,
@@ -1238,7 +1242,7 @@ bool prefill_frags_fusable(uint32_t num_prev, uint32_t head_dim, uint32_t gqa) {
 int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const float *vc, const uint32_t *slots,
                         uint32_t n_tok, uint32_t num_prev, uint32_t num_q_heads, uint32_t head_dim, uint32_t kv_dim,
                         uint32_t gqa, float scale, uint32_t window, float *out, __bf16 *outb, float *ws,
-                        unsigned char *frag, size_t frag_bytes, bool new_frags_ready) {
+                        unsigned char *frag, size_t frag_bytes, bool new_frags_ready, uint32_t ntt) {
     if (head_dim == 256 && (gqa == 1 || gqa == 2 || gqa == 4 || gqa == 8)) {
         // the keys' operand fragments, chunks c_lo .. c_hi - 1; those of the
         // new tokens' chunks may be written already (by the rope kernel)
@@ -1269,7 +1273,7 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
         const dim3 mgrid(num_q_heads / gqa, items);
 #define CHN_PATTN_MF(G)                                                                                  \
     k_prefill_attn_mf<G><<<mgrid, 64 * kPaWaves, 0, st>>>(q, frag, c_lo, nfch, num_prev, n_tok, num_q_heads, scale, \
-                                                         window, out, outb, ws, geo.maxparts)
+                                                         window, out, outb, ws, geo.maxparts, ntt)
         switch (gqa) {
         case 1: CHN_PATTN_MF(1); break;
         case 2: CHN_PATTN_MF(2); break;
@@ -1280,14 +1284,14 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
         if (split_tiles) {
             const size_t nrow = (size_t)n_tok * num_q_heads, nq4 = nrow * head_dim / 4;
             k_prefill_attn_merge<<<(unsigned)((nq4 + 255) / 256), 256, 0, st>>>(ws, geo, num_q_heads, nrow, head_dim,
-                                                                                  out, outb);
+                                                                                  out, outb, ntt);
         }
         return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
     }
     dim3 grid(n_tok, num_q_heads / gqa);
 #define CHN_PATTN(DV, G) \
     k_prefill_attn<DV, G><<<grid, 256, 0, st>>>(q, kc, vc, slots, num_prev, num_q_heads, kv_dim, scale, window, out, \
-                                                outb)
+                                                outb, ntt)
     if (head_dim == 256) {
         switch (gqa) {
         case 1: CHN_PATTN(1, 1); break;

@@ -93,11 +93,12 @@ int launch_rmsnorm(hipStream_t s, float *x, const float *r, const float *w, floa
 // nparts (1, 2 or 4) partial outputs r + p * pstride of a split
 // contraction, added in index order; with post_w, r' = rmsnorm(branch) *
 // post_w (else r' = branch); with add, x = (x + r') * scalar (written
-// back); y = rmsnorm(x) * w as bf16 into yb and, if y != NULL, as fp32.
+// back); y = rmsnorm(x) * w as bf16 into yb (xb_at order for ntt) and, if
+// y != NULL, as fp32.
 // The same arithmetic, in the same order, as launch_rmsnorm's two passes.
 int launch_rmsnorm_chain(hipStream_t s, float *x, const float *r, const float *post_w, const float *w, __bf16 *yb,
                          float *y, uint32_t dim, uint32_t rows, float eps, float scalar, bool add,
-                         uint32_t nparts = 1, size_t pstride = 0);
+                         uint32_t nparts = 1, size_t pstride = 0, uint32_t ntt = 0);
 // Digit planes of x (nb 32-blocks) into xp (xplanes_bytes(nb)).
 int launch_xplanes(hipStream_t s, const float *x, uint32_t *xp, uint32_t nb);
 
@@ -220,7 +221,8 @@ int launch_rope_decode_attn(chn_ctx *ctx, const float *q_in, const float *k_in, 
                             uint32_t kv_dim, uint32_t gqa, uint32_t rot, int k_eq_v, const float2 *rope_tab,
                             float eps, float scale, float *out, float *ws, uint32_t *xp,
                             const uint32_t *skip = nullptr);
-// out: [n_tok][num_q_heads * head_dim] fp32, or bf16 into outb when set.
+// out: [n_tok][num_q_heads * head_dim] fp32, or bf16 into outb (xb_at order
+// for ntt) when set.
 // ws (prefill_attn_ws_bytes, or NULL): lets short prompts split each query
 // tile's keys between two workgroups.  frag (prefill_frag_bytes for the
 // KV heads and num_prev + n_tok keys): the keys' bf16 operand fragments,
@@ -233,7 +235,7 @@ bool prefill_frags_fusable(uint32_t num_prev, uint32_t head_dim, uint32_t gqa);
 int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const float *vc, const uint32_t *slots,
                         uint32_t n_tok, uint32_t num_prev, uint32_t num_q_heads, uint32_t head_dim, uint32_t kv_dim,
                         uint32_t gqa, float scale, uint32_t window, float *out, __bf16 *outb, float *ws,
-                        unsigned char *frag, size_t frag_bytes, bool new_frags_ready = false);
+                        unsigned char *frag, size_t frag_bytes, bool new_frags_ready = false, uint32_t ntt = 0);
 size_t xbytes_bytes(uint32_t nb);
 int launch_gemv_q8(hipStream_t st, const uint32_t *W, const float *x, float *y, uint32_t M, uint32_t nb,
                    uint32_t *xp_ws);
@@ -257,9 +259,42 @@ int launch_topk64(hipStream_t st, const float *logits, uint32_t V, uint32_t *ids
 int launch_embed(hipStream_t st, const uint16_t *table, const uint32_t *tokens, uint32_t n, uint32_t H, float scale,
                  float *x);
 int launch_quantize(hipStream_t st, int q8, const uint16_t *src, uint32_t *dst, uint64_t nblk);
+// Contractions of at most kFewTokens tokens run on gemm_q4_few.hip, whose
+// bf16 activations lie in operand order (xb_at); larger ones read them row
+// by row.  At 128 tokens the few-token kernels lead or tie on every 12B shape
+// (gate/up 77 against 118 us, down 51 / 57, q/k/v 20 / 31, o_proj 18 / 20);
+// at 192 they trail on down (76 / 59) and o_proj (26 / 22).
+constexpr uint32_t kFewTokens = 128;
+inline bool few_tokens(uint32_t n_tok) { return n_tok <= kFewTokens; }
+inline uint32_t xb_tiles(uint32_t n_tok) { return (n_tok + 15) / 16; }
+// Tile count to pass as xb_at's ntt for a contraction of n_tok tokens.
+inline uint32_t xb_layout(uint32_t n_tok) { return few_tokens(n_tok) ? xb_tiles(n_tok) : 0u; }
+// Elements of the bf16 activation buffer of n_tok tokens of width K.
+inline size_t xb_elems(uint32_t n_tok, uint32_t K) {
+    return few_tokens(n_tok) ? (size_t)xb_tiles(n_tok) * 16 * ((K + 255) / 256) * 256 : (size_t)n_tok * K;
+}
+// Element (token t, k) of bf16 activations of `width` columns: row-major
+// when ntt is 0, else operand order of k_q4gemm_few over ntt tiles of 16
+// tokens: per 256 K, per half h (the 32-blocks 2g + h), per tile, per word j
+// of the blocks, 64 lanes (16 g + t % 16) of 8 consecutive k.  Eight aligned
+// k of a token stay together.
+__host__ __device__ inline size_t xb_at(uint32_t ntt, uint32_t width, uint32_t t, uint32_t k) {
+    if (!ntt) return (size_t)t * width + k;
+    const uint32_t half = (k >> 8) * 2 + ((k >> 5) & 1), g = (k >> 6) & 3, j = (k >> 3) & 3;
+    return ((((size_t)half * ntt + (t >> 4)) * 4 + j) * 64 + g * 16 + (t & 15)) * 8 + (k & 7);
+}
+int launch_to_bf16_few(hipStream_t st, const float *X, __bf16 *xb, uint32_t n_tok, uint32_t K);
+// nseg matrices over the same activations (nmat 1), or gate W[0] and up W1
+// (nmat 2).  Yb (nmat 2): the result as bf16 instead of Y[0], in xb_at order
+// when yb_frag, else row-major.
+int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1, float *const *Y,
+                      const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked,
+                      __bf16 *Yb = nullptr, bool yb_frag = false);
 // W0/W1 in the reference Q4 layout, or in Q4R with repacked.  X (fp32) is
-// converted into xb; with X == NULL, xb already holds the bf16 activations.
-// Yb (two-matrix form only): the result goes to Yb as bf16 instead of Y.
+// converted into xb (xb_elems); with X == NULL, xb already holds the bf16
+// activations, in xb_at order for xb_layout(n_tok).
+// Yb (two-matrix form only): the result goes to Yb as bf16 instead of Y,
+// in the next contraction's order when X == NULL, else row-major.
 // po (single matrix): a shape that splits K may store its partial sums to
 // Y + p * po->stride, p < po->max_parts (1, 2 or 4), with plain stores
 // instead of clearing Y and adding into it; po->parts tells how many it

@@ -1,6 +1,7 @@
 // Batched prefill contractions over Q4 weights on gfx950 MFMA:
 // batch_gemm_q4 (shaders/batch_gemm_q4.wgsl) and batch_fused_mlp_q4
-// (shaders/batch_fused_mlp_q4.wgsl).
+// (shaders/batch_fused_mlp_q4.wgsl), for more than kFewTokens tokens
+// (gemm_q4_few.hip serves fewer).
 //
 //   Y[t, n] = sum_k X[t, k] * W[n, k]        (t < n_tok, n < M)
 //
@@ -1126,6 +1127,13 @@ int launch_q4gemm(chn_ctx *ctx, int nmat, const float *X, const uint32_t *W0, co
     const size_t n = X ? (size_t)n_tok * K : 0;
     GemmArgs a{xb, W0, W1, Y, n_tok, M, K};
     if (po) po->parts = 1;
+    if (few_tokens(n_tok)) {
+        if (Yb && nmat == 1) return set_err(ctx, CHN_E_UNSUPPORTED, "bf16 output needs the two-matrix contraction");
+        if (n && launch_to_bf16_few(ctx->stream, X, xb, n_tok, K)) return hip_fail(ctx, hipGetLastError(), "k_to_bf16_few");
+        if (launch_q4gemm_few(ctx->stream, nmat, 1, &W0, W1, &Y, &M, n_tok, K, xb, repacked, Yb, Yb && !X))
+            return hip_fail(ctx, hipGetLastError(), "k_q4gemm_few");
+        return CHN_OK;
+    }
     if (nmat == 1 && K % 64 == 0 && po && po->max_parts >= 4 && split4_fits(n_tok, M, K)) {
         if (Yb) return set_err(ctx, CHN_E_UNSUPPORTED, "bf16 output needs the two-matrix contraction");
         if (n) {
@@ -1189,6 +1197,15 @@ int launch_q4gemm(chn_ctx *ctx, int nmat, const float *X, const uint32_t *W0, co
 int launch_q4gemm_qkv(chn_ctx *ctx, const float *X, const uint32_t *Wq, const uint32_t *Wk, const uint32_t *Wv,
                       float *Yq, float *Yk, float *Yv, uint32_t n_tok, uint32_t Mq, uint32_t Mkv, uint32_t K,
                       __bf16 *xb) {
+    if (few_tokens(n_tok)) {
+        const uint32_t *const W[3] = {Wq, Wk, Wv};
+        float *const Y[3] = {Yq, Yk, Yv};
+        const uint32_t M[3] = {Mq, Mkv, Mkv};
+        if (X && launch_to_bf16_few(ctx->stream, X, xb, n_tok, K)) return hip_fail(ctx, hipGetLastError(), "k_to_bf16_few");
+        if (launch_q4gemm_few(ctx->stream, 1, 3, W, nullptr, Y, M, n_tok, K, xb, true))
+            return hip_fail(ctx, hipGetLastError(), "k_q4gemm_few");
+        return CHN_OK;
+    }
     if (K % 64 != 0) {
         int rc = launch_q4gemm(ctx, 1, X, Wq, nullptr, Yq, n_tok, Mq, K, xb, true);
         if (!rc) rc = launch_q4gemm(ctx, 1, nullptr, Wk, nullptr, Yk, n_tok, Mkv, K, xb, true);
@@ -1222,7 +1239,7 @@ static int gemm_common(chn_ctx *ctx, int nmat, const uint32_t *W0, const uint32_
     CHN_REQUIRE(ctx, aligned(W0, repacked ? 16 : 4) && (!W1 || aligned(W1, repacked ? 16 : 4)),
                 "weights must be %d-byte aligned", repacked ? 16 : 4);
     if (!n_tok || !M) return CHN_OK;
-    int rc = ensure_workspace(ctx, (size_t)n_tok * K * 2);
+    int rc = ensure_workspace(ctx, xb_elems(n_tok, K) * 2);
     if (rc) return rc;
     return launch_q4gemm(ctx, nmat, X, W0, W1, Y, n_tok, M, K, (__bf16 *)ctx->ws, repacked, Yb);
 }
@@ -1267,7 +1284,7 @@ extern "C" int chn_batch_qkv_q4r(chn_ctx *ctx, const void *Wq, const void *Wk, c
     CHN_REQUIRE(ctx, K > 0 && K % 32 == 0, "K=%u must be a positive multiple of 32", K);
     CHN_REQUIRE(ctx, aligned(X, 16) && aligned(Wq, 16) && aligned(Wk, 16) && aligned(Wv, 16), "misaligned argument");
     if (!n_tok || !q_dim || !kv_dim) return CHN_OK;
-    int rc = ensure_workspace(ctx, (size_t)n_tok * K * 2);
+    int rc = ensure_workspace(ctx, xb_elems(n_tok, K) * 2);
     if (rc) return rc;
     return launch_q4gemm_qkv(ctx, X, (const uint32_t *)Wq, (const uint32_t *)Wk, (const uint32_t *)Wv, Yq, Yk, Yv,
                              n_tok, q_dim, kv_dim, K, (__bf16 *)ctx->ws);

@@ -212,8 +212,15 @@ static int alloc_runtime(chn_model *m) {
     m->pfrag_bytes = prefill_frag_bytes(md.kvd / 256 ? md.kvd / 256 : 1, kSlotsMax + T);
     M_ALLOC(m->pfrag, m->pfrag_bytes);
     M_ALLOC(m->prope, (size_t)2 * T * kRopePairs * sizeof(float2));
-    M_ALLOC(m->pact, (size_t)T * I * 4);
-    M_ALLOC(m->pxb, (size_t)T * (H > qd ? H : qd) * 2);   // bf16 operands of width H or qd; act goes to pact
+    // bf16 operands: width I in pact, H or qd in pxb.  Few-token prefills pad
+    // tokens to 16 and K to 256 (xb_elems); larger ones take n * K.
+    const uint32_t Tf = T < kFewTokens ? T : kFewTokens, W = H > qd ? H : qd;
+    auto xb_bytes = [&](uint32_t K) {
+        const size_t rows = (size_t)T * K, few = xb_elems(Tf, K);
+        return 2 * (rows > few ? rows : few);
+    };
+    M_ALLOC(m->pact, xb_bytes(I));
+    M_ALLOC(m->pxb, xb_bytes(W));
     M_ALLOC(m->pslots, (size_t)(kSlotsMax + T) * 4);
     M_ALLOC(m->ptok, (size_t)T * 4);
     hipError_t e = hipHostMalloc((void **)&m->h_x, H * 4);
@@ -882,8 +889,10 @@ extern "C" int chn_prefill(chn_model *m, const uint32_t *tokens, uint32_t n, con
     // directly: the norm chains and the attention into pxb, gate/up into the
     // act buffer (as bf16).  Where o_proj and down split K, their partial
     // sums go to pmlp + p * max_tok * H and the next norm chain adds them.
+    // Both lie in the order the contractions of n tokens read (xb_at).
     __bf16 *xb = m->pxb;
     __bf16 *actb = (__bf16 *)m->pact;
+    const uint32_t ntt = xb_layout(n);
     // the prompt's rotation angles, once per kind (sliding / full layers)
     const HeadShape hs[2] = {head_shape(c, false), head_shape(c, true)};
     const float thetas[2] = {c.rope_theta, c.rope_theta_full};
@@ -893,7 +902,8 @@ extern "C" int chn_prefill(chn_model *m, const uint32_t *tokens, uint32_t n, con
         const auto &l = m->L[i];
         const float theta = l.full ? c.rope_theta_full : c.rope_theta;
         if (i == 0)
-            P_(launch_rmsnorm_chain(s, m->px, nullptr, nullptr, l.in_norm, xb, nullptr, H, n, eps, 1.0f, false));
+            P_(launch_rmsnorm_chain(s, m->px, nullptr, nullptr, l.in_norm, xb, nullptr, H, n, eps, 1.0f, false, 1, 0,
+                                      ntt));
         const uint32_t D = l.D, nkv = l.nkv, qd = l.qd, kvd = l.kvd, gqa = l.gqa;
         P_(launch_q4gemm_qkv(ctx, nullptr, l.Wq, l.Wk, l.Wv, m->pq, m->pk, m->pv, n, qd, kvd, H, xb));
         // sliding layers see the last 1024 slots (shaders/batch_causal_attn.wgsl:53)
@@ -906,19 +916,19 @@ extern "C" int chn_prefill(chn_model *m, const uint32_t *tokens, uint32_t n, con
                                  num_prev_slots, start_clock, n, nq, nkv, D, l.rot, (int)c.k_eq_v, theta, eps,
                                  ptab[l.full ? 1 : 0], fuse ? m->pfrag : nullptr, m->pfrag_bytes, win));
         P_(launch_prefill_attn(s, m->pq, l.kc, l.vc, m->pslots, n, num_prev_slots, nq, D, kvd, gqa, 1.0f, win,
-                               nullptr, xb, m->pattn_ws, m->pfrag, m->pfrag_bytes, fuse));
+                               nullptr, xb, m->pattn_ws, m->pfrag, m->pfrag_bytes, fuse, ntt));
         const size_t pstride = (size_t)m->max_tok * H;
         PartialOut po_o{pstride, 2};
         P_(launch_q4gemm(ctx, 1, nullptr, l.Wo, nullptr, m->pmlp, n, H, qd, xb, true, nullptr, &po_o));
         P_(launch_rmsnorm_chain(s, m->px, m->pmlp, l.has_post_attn ? l.post_attn : nullptr, l.pre_ffn, xb, nullptr,
-                                H, n, eps, 1.0f, true, po_o.parts, pstride));
+                                H, n, eps, 1.0f, true, po_o.parts, pstride, ntt));
         P_(launch_q4gemm(ctx, 2, nullptr, l.Wg, l.Wu, nullptr, n, I, H, xb, true, actb));
         PartialOut po_d{pstride, 4};
         P_(launch_q4gemm(ctx, 1, nullptr, l.Wd, nullptr, m->pmlp, n, H, I, actb, true, nullptr, &po_d));
         const bool last = i + 1 == c.num_layers;
         const float *next_norm = last ? m->final_norm : m->L[i + 1].in_norm;
         P_(launch_rmsnorm_chain(s, m->px, m->pmlp, l.has_post_ffn ? l.post_ffn : nullptr, next_norm, xb,
-                                last ? m->pn : nullptr, H, n, eps, l.scalar, true, po_d.parts, pstride));
+                                last ? m->pn : nullptr, H, n, eps, l.scalar, true, po_d.parts, pstride, ntt));
         if ((i + 1) % 4 == 0 || i + 1 == c.num_layers) {
             if (i + 1 == c.num_layers && (logits_out || topk_ids)) {
                 CHN_HIP(ctx, hipMemcpyAsync(m->normed, m->pn + (size_t)(n - 1) * H, H * 4, hipMemcpyDeviceToDevice, s));

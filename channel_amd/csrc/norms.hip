@@ -75,7 +75,7 @@ template <bool POST, bool ADD, int NP>
 __global__ __launch_bounds__(256) void k_rmsnorm_chain(float *__restrict__ x, const float *__restrict__ r, size_t ps,
                                                        const float *__restrict__ pw, const float *__restrict__ w,
                                                        __bf16 *__restrict__ yb, float *__restrict__ y, uint32_t dim,
-                                                       float eps, float scalar) {
+                                                       float eps, float scalar, uint32_t ntt) {
     __shared__ float sh[4];
     const size_t off = (size_t)blockIdx.x * dim;
     f4n *xr = (f4n *)(x + off);
@@ -114,8 +114,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_chain(float *__restrict__ x, co
     for (uint32_t i = threadIdx.x; i < dv; i += 256) {
         const f4n o = (xr[i] * inv) * wr[i];
         bf16x2 lo = {(__bf16)o.x, (__bf16)o.y}, hi = {(__bf16)o.z, (__bf16)o.w};
-        *(bf16x2 *)(yb + off + 4 * (size_t)i) = lo;
-        *(bf16x2 *)(yb + off + 4 * (size_t)i + 2) = hi;
+        __bf16 *yo = yb + xb_at(ntt, dim, blockIdx.x, 4 * i);
+        *(bf16x2 *)yo = lo;
+        *(bf16x2 *)(yo + 2) = hi;
         if (y) *(f4n *)(y + off + 4 * (size_t)i) = o;
     }
 }
@@ -129,7 +130,7 @@ template <bool POST, bool ADD, int NP>
 __global__ __launch_bounds__(256) void k_rmsnorm_chain_r(float *__restrict__ x, const float *__restrict__ r, size_t ps,
                                                          const float *__restrict__ pw, const float *__restrict__ w,
                                                          __bf16 *__restrict__ yb, float *__restrict__ y, uint32_t dim,
-                                                         float eps, float scalar) {
+                                                         float eps, float scalar, uint32_t ntt) {
     constexpr int NPT = 4;
     __shared__ float sh[4];
     const size_t off = (size_t)blockIdx.x * dim;
@@ -187,8 +188,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_chain_r(float *__restrict__ x, 
         if (i >= dv) continue;
         const f4n o = (xv[k] * inv) * wv[k];
         bf16x2 lo = {(__bf16)o.x, (__bf16)o.y}, hi = {(__bf16)o.z, (__bf16)o.w};
-        *(bf16x2 *)(yb + off + 4 * (size_t)i) = lo;
-        *(bf16x2 *)(yb + off + 4 * (size_t)i + 2) = hi;
+        __bf16 *yo = yb + xb_at(ntt, dim, blockIdx.x, 4 * i);
+        *(bf16x2 *)yo = lo;
+        *(bf16x2 *)(yo + 2) = hi;
         if (y) *(f4n *)(y + off + 4 * (size_t)i) = o;
     }
 }
@@ -204,7 +206,7 @@ template <bool POST, bool ADD, int NP>
 __global__ __launch_bounds__(256) void k_rmsnorm_chain_p(float *__restrict__ x, const float *__restrict__ r, size_t ps,
                                                          const float *__restrict__ pw, const float *__restrict__ w,
                                                          __bf16 *__restrict__ yb, float *__restrict__ y, uint32_t dim,
-                                                         uint32_t rows, float eps, float scalar) {
+                                                         uint32_t rows, float eps, float scalar, uint32_t ntt) {
     constexpr int NPT = 4;
     __shared__ float sh[4];
     const f4n *pwr = (const f4n *)pw;
@@ -291,8 +293,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_chain_p(float *__restrict__ x, 
             if (i >= dv) continue;
             const f4n o = (xv[k] * inv) * wv[k];
             bf16x2 lo = {(__bf16)o.x, (__bf16)o.y}, hi = {(__bf16)o.z, (__bf16)o.w};
-            *(bf16x2 *)(yb + off + 4 * (size_t)i) = lo;
-            *(bf16x2 *)(yb + off + 4 * (size_t)i + 2) = hi;
+            __bf16 *yo = yb + xb_at(ntt, dim, row, 4 * i);
+            *(bf16x2 *)yo = lo;
+            *(bf16x2 *)(yo + 2) = hi;
             if (y) *(f4n *)(y + off + 4 * (size_t)i) = o;
         }
     };
@@ -312,28 +315,28 @@ __global__ __launch_bounds__(256) void k_rmsnorm_chain_p(float *__restrict__ x, 
 template <bool POST, bool ADD, int NP>
 static void launch_chain_kind(hipStream_t s, float *x, const float *r, size_t ps, const float *post_w,
                               const float *w, __bf16 *yb, float *y, uint32_t dim, uint32_t rows, float eps,
-                              float scalar) {
+                              float scalar, uint32_t ntt) {
     if (dim <= 4096 && rows > kChainGrid)
-        k_rmsnorm_chain_p<POST, ADD, NP><<<kChainGrid, 256, 0, s>>>(x, r, ps, post_w, w, yb, y, dim, rows, eps, scalar);
+        k_rmsnorm_chain_p<POST, ADD, NP><<<kChainGrid, 256, 0, s>>>(x, r, ps, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
     else if (dim <= 4096)
-        k_rmsnorm_chain_r<POST, ADD, NP><<<rows, 256, 0, s>>>(x, r, ps, post_w, w, yb, y, dim, eps, scalar);
-    else k_rmsnorm_chain<POST, ADD, NP><<<rows, 256, 0, s>>>(x, r, ps, post_w, w, yb, y, dim, eps, scalar);
+        k_rmsnorm_chain_r<POST, ADD, NP><<<rows, 256, 0, s>>>(x, r, ps, post_w, w, yb, y, dim, eps, scalar, ntt);
+    else k_rmsnorm_chain<POST, ADD, NP><<<rows, 256, 0, s>>>(x, r, ps, post_w, w, yb, y, dim, eps, scalar, ntt);
 }
 
 template <int NP>
 static void launch_chain_np(hipStream_t s, float *x, const float *r, size_t ps, const float *post_w, const float *w,
-                            __bf16 *yb, float *y, uint32_t dim, uint32_t rows, float eps, float scalar) {
-    if (post_w) launch_chain_kind<true, true, NP>(s, x, r, ps, post_w, w, yb, y, dim, rows, eps, scalar);
-    else launch_chain_kind<false, true, NP>(s, x, r, ps, post_w, w, yb, y, dim, rows, eps, scalar);
+                            __bf16 *yb, float *y, uint32_t dim, uint32_t rows, float eps, float scalar, uint32_t ntt) {
+    if (post_w) launch_chain_kind<true, true, NP>(s, x, r, ps, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
+    else launch_chain_kind<false, true, NP>(s, x, r, ps, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
 }
 
 int launch_rmsnorm_chain(hipStream_t s, float *x, const float *r, const float *post_w, const float *w, __bf16 *yb,
                          float *y, uint32_t dim, uint32_t rows, float eps, float scalar, bool add, uint32_t nparts,
-                         size_t pstride) {
-    if (!add) launch_chain_kind<false, false, 1>(s, x, r, 0, post_w, w, yb, y, dim, rows, eps, scalar);
-    else if (nparts == 4) launch_chain_np<4>(s, x, r, pstride, post_w, w, yb, y, dim, rows, eps, scalar);
-    else if (nparts == 2) launch_chain_np<2>(s, x, r, pstride, post_w, w, yb, y, dim, rows, eps, scalar);
-    else if (nparts == 1) launch_chain_np<1>(s, x, r, 0, post_w, w, yb, y, dim, rows, eps, scalar);
+                         size_t pstride, uint32_t ntt) {
+    if (!add) launch_chain_kind<false, false, 1>(s, x, r, 0, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
+    else if (nparts == 4) launch_chain_np<4>(s, x, r, pstride, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
+    else if (nparts == 2) launch_chain_np<2>(s, x, r, pstride, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
+    else if (nparts == 1) launch_chain_np<1>(s, x, r, 0, post_w, w, yb, y, dim, rows, eps, scalar, ntt);
     else return CHN_E_UNSUPPORTED;
     return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
 }
