@@ -24,7 +24,6 @@
 
 namespace chn {
 
-constexpr int kAttnChunk = 64;     // prefill: slots per online-softmax step
 constexpr uint32_t kDecGrid = 32;  // decode: workgroups per KV head (at most)
 constexpr int kMaxChunks = 8;      // decode: 16-entry chunks per split at most (4096 / 16 / kDecGrid)
 static_assert(kMaxChunks * 16 * kDecGrid >= 4096, "a split's chunks of the largest list");
@@ -56,139 +55,6 @@ constexpr uint32_t kPaPartChunks = 4;
 constexpr int kPaWaves = 8;
 size_t prefill_attn_ws_bytes(uint32_t n_tok, uint32_t num_q_heads, uint32_t head_dim) {
     return kPaParts * (size_t)n_tok * num_q_heads * ((size_t)head_dim + 2) * 4;
-}
-
-// Running softmax state of one lane: lane row r = lane / 16 holds slots
-// r, r+4, r+8, r+12 of each wave's 16, column c = lane % 16 holds 16*DV
-// consecutive dims, so one slot's row (1 KB at D = 256) is read by a
-// 16-lane row as 64 contiguous bytes per lane and its score reduces inside
-// the row with DPP.
-template <int DV, int GQA>
-struct AttnState {
-    float M[GQA], l[GQA];
-    f4 acc[GQA][4 * DV];
-};
-
-// One 64-slot chunk [c0, c0 + cnt) of the list for KV head kvh: scores,
-// running max / sum update (rescaling the accumulators), p-weighted V.
-template <int DV, int GQA>
-__device__ __forceinline__ void attn_chunk(AttnState<DV, GQA> &st, const f4 (&q)[GQA][4 * DV],
-                                           const float *__restrict__ Kc, const float *__restrict__ Vc,
-                                           const uint32_t *__restrict__ slots, uint32_t c0, uint32_t cnt,
-                                           uint32_t kv_dim, uint32_t kvh, float scale, float (&sc)[GQA][kAttnChunk]) {
-    constexpr int D = DV * 256;
-    constexpr int NF = 4 * DV;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r = lane >> 4, c = lane & 15;
-    const uint32_t base = c0 + wave * 16;
-    const uint32_t nval = cnt > (uint32_t)(wave * 16) ? cnt - wave * 16 : 0;
-    const uint32_t my_slot = (uint32_t)lane < nval && lane < 16 ? slots[base + lane] : 0u;
-    const size_t dim0 = (size_t)kvh * D + (size_t)c * NF * 4;
-
-    f4 kr[4][NF], vr[4][NF];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int i = r + 4 * u;
-        const uint32_t ps = (uint32_t)__shfl(my_slot, i, 64);
-        const bool ok = (uint32_t)i < nval;
-        const float *kp = Kc + (size_t)ps * kv_dim + dim0;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) kr[u][f] = ok ? *(const f4 *)(kp + 4 * f) : f4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int i = r + 4 * u;
-        const uint32_t ps = (uint32_t)__shfl(my_slot, i, 64);
-        const bool ok = (uint32_t)i < nval;
-        const float *vp = Vc + (size_t)ps * kv_dim + dim0;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) vr[u][f] = ok ? *(const f4 *)(vp + 4 * f) : f4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int h = 0; h < GQA; ++h) {
-            float d = 0.0f;
-#pragma unroll
-            for (int f = 0; f < NF; ++f) {
-                d = fmaf(q[h][f].x, kr[u][f].x, d);
-                d = fmaf(q[h][f].y, kr[u][f].y, d);
-                d = fmaf(q[h][f].z, kr[u][f].z, d);
-                d = fmaf(q[h][f].w, kr[u][f].w, d);
-            }
-            d = row16_sum(d);
-            if (c == 0) sc[h][wave * 16 + r + 4 * u] = d * scale;
-        }
-    __syncthreads();
-    float p[GQA];
-#pragma unroll
-    for (int h = 0; h < GQA; ++h) {
-        const float sv = (uint32_t)lane < cnt ? sc[h][lane] : kNegBig;
-        const float Mn = fmaxf(st.M[h], wave_max64(sv));
-        const float e = (uint32_t)lane < cnt ? expf(sv - Mn) : 0.0f;
-        const float rs = expf(st.M[h] - Mn);
-        st.l[h] = st.l[h] * rs + wave_sum64(e);
-#pragma unroll
-        for (int f = 0; f < NF; ++f) st.acc[h][f] *= rs;
-        st.M[h] = Mn;
-        p[h] = e;
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int h = 0; h < GQA; ++h) sc[h][lane] = p[h];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int i = r + 4 * u;
-        if ((uint32_t)i < nval) {
-#pragma unroll
-            for (int h = 0; h < GQA; ++h) {
-                const float pw = sc[h][wave * 16 + i];
-#pragma unroll
-                for (int f = 0; f < NF; ++f) st.acc[h][f] += pw * vr[u][f];
-            }
-        }
-    }
-    __syncthreads();   // sc is rewritten by the next chunk
-}
-
-// Sum the 16 (wave, row) partial accumulators of each head in a fixed order
-// and hand each finished float4 column to `emit(head, column, value)`.
-template <int DV, int GQA, typename Emit>
-__device__ __forceinline__ void attn_reduce(const AttnState<DV, GQA> &st, f4 (*pacc)[GQA < 2 ? GQA : 2][64 * DV],
-                                            Emit emit) {
-    constexpr int NF = 4 * DV;
-    constexpr int HC = GQA < 2 ? GQA : 2;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r = lane >> 4, c = lane & 15;
-#pragma unroll
-    for (int h0 = 0; h0 < GQA; h0 += HC) {
-#pragma unroll
-        for (int hh = 0; hh < HC; ++hh)
-#pragma unroll
-            for (int f = 0; f < NF; ++f) pacc[wave * 4 + r][hh][c * NF + f] = st.acc[h0 + hh][f];
-        __syncthreads();
-        for (int idx = threadIdx.x; idx < HC * 16 * NF; idx += 256) {
-            const int hh = idx / (16 * NF), col = idx % (16 * NF);
-            f4 t = pacc[0][hh][col];
-#pragma unroll
-            for (int j = 1; j < 16; ++j) t += pacc[j][hh][col];
-            emit(h0 + hh, col, t);
-        }
-        __syncthreads();
-    }
-}
-
-template <int DV, int GQA>
-__device__ __forceinline__ void load_q(f4 (&q)[GQA][4 * DV], const float *__restrict__ Q, uint32_t qh0) {
-    constexpr int D = DV * 256;
-    const int c = threadIdx.x & 15;
-#pragma unroll
-    for (int h = 0; h < GQA; ++h)
-#pragma unroll
-        for (int f = 0; f < 4 * DV; ++f) q[h][f] = *(const f4 *)(Q + (size_t)(qh0 + h) * D + c * 16 * DV + 4 * f);
 }
 
 // Inputs of the fused per-head RMSNorm + RoPE of the decode step
@@ -711,50 +577,12 @@ __device__ __forceinline__ void store_out4(float *out, __bf16 *outb, uint32_t nt
     }
 }
 
-// Prefill (shaders/batch_causal_attn.wgsl): one workgroup per (token, KV
-// head) walks slots [start, prev + t + 1) of the list in 64-slot chunks with
-// an online softmax; start = S - window for window > 0 and S > window.
-template <int DV, int GQA>
-__global__ __launch_bounds__(256) void k_prefill_attn(const float *__restrict__ Q, const float *__restrict__ Kc,
-                                                      const float *__restrict__ Vc,
-                                                      const uint32_t *__restrict__ slots, uint32_t num_prev,
-                                                      uint32_t num_q_heads, uint32_t kv_dim, float scale,
-                                                      uint32_t window, float *__restrict__ out,
-                                                      __bf16 *__restrict__ outb, uint32_t ntt) {
-    constexpr int D = DV * 256;
-    const uint32_t t = blockIdx.x, kvh = blockIdx.y;
-    const uint32_t S = num_prev + t + 1;
-    const uint32_t start = (window > 0 && S > window) ? S - window : 0;
-    __shared__ float sc[GQA][kAttnChunk];
-    __shared__ f4 pacc[16][GQA < 2 ? GQA : 2][64 * DV];
-    const size_t q_row = (size_t)t * num_q_heads * D;
-    f4 q[GQA][4 * DV];
-    load_q<DV, GQA>(q, Q + q_row, kvh * GQA);
-    AttnState<DV, GQA> st;
-#pragma unroll
-    for (int h = 0; h < GQA; ++h) {
-        st.M[h] = -1e9f;
-        st.l[h] = 0.0f;
-#pragma unroll
-        for (int f = 0; f < 4 * DV; ++f) st.acc[h][f] = f4{0, 0, 0, 0};
-    }
-    for (uint32_t c0 = start; c0 < S; c0 += kAttnChunk) {
-        const uint32_t cnt = (S - c0 < (uint32_t)kAttnChunk) ? S - c0 : kAttnChunk;
-        attn_chunk<DV, GQA>(st, q, Kc, Vc, slots, c0, cnt, kv_dim, kvh, scale, sc);
-    }
-    float inv[GQA];
-#pragma unroll
-    for (int h = 0; h < GQA; ++h) inv[h] = 1.0f / (st.l[h] + 1e-9f);
-    attn_reduce<DV, GQA>(st, pacc, [&](int h, int col, f4 v) {
-        store_out4(out, outb, ntt, num_q_heads * D, t, (kvh * GQA + h) * D + 4 * col, v * inv[h]);
-    });
-}
-
 // ---------------------------------------------------------------------
 // Prefill attention on the matrix cores, head_dim 256.
 //
-// Same result as k_prefill_attn (an online softmax over each query's causal
-// window), computed per workgroup for 64 query rows (64 / GQA tokens x the
+// An online softmax over each query's causal window (shaders/
+// batch_causal_attn.wgsl: keys [start, prev + t + 1) of the list, start = S -
+// window for window > 0 and S > window), computed per workgroup for 64 query rows (64 / GQA tokens x the
 // GQA heads of one KV head) against 32-key chunks of the slot list:
 //  * scores are formed transposed, S^T = K Q^T, with
 //    v_mfma_f32_16x16x32_bf16; each fp32 operand is split into bf16 high
@@ -897,10 +725,44 @@ __host__ __device__ inline uint32_t pa_parts(const PaGeom &g, uint32_t tile) {
     return np < 1 ? 1 : (np > g.maxparts ? g.maxparts : np);
 }
 
+// Work item `it` of a KV head: part `part` of the nparts of query tile
+// `tile`, the tiles' parts numbered in tile order; every wave finds it with a
+// prefix sum of the tiles' part counts over the lanes.
+__device__ __forceinline__ void pa_item(const PaGeom &geo, uint32_t it, int lane, uint32_t &tile, uint32_t &part,
+                                        uint32_t &nparts) {
+    tile = 0;
+    part = 0;
+    nparts = 1;
+    const uint32_t ntiles = (geo.n_tok + geo.TQ - 1) / geo.TQ;
+    uint32_t base = 0;
+    for (uint32_t t0 = 0; t0 < ntiles; t0 += 64) {
+        const uint32_t t = t0 + lane;
+        const uint32_t np = t < ntiles ? pa_parts(geo, t) : 0u;
+        uint32_t incl = np;                                    // inclusive prefix sum over the lanes
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const uint32_t v = (uint32_t)__shfl_up((int)incl, d, 64);
+            incl += lane >= d ? v : 0u;
+        }
+        const uint32_t total = (uint32_t)__shfl((int)incl, 63, 64);
+        if (it < base + total) {
+            const uint32_t r = it - base;
+            const uint64_t hit = __ballot(r < incl && r >= incl - np);
+            const int L = __builtin_ctzll(hit);
+            tile = t0 + L;
+            nparts = (uint32_t)__shfl((int)np, L, 64);
+            part = r - ((uint32_t)__shfl((int)incl, L, 64) - nparts);
+            break;
+        }
+        base += total;
+    }
+    tile = __builtin_amdgcn_readfirstlane(tile);
+    part = __builtin_amdgcn_readfirstlane(part);
+    nparts = __builtin_amdgcn_readfirstlane(nparts);
+}
+
 // F: the pre-pass output for chunks c_lo .. c_lo + nfch - 1.  Grid (KV
-// heads, work items): item `it` of a KV head is part `part` of query tile
-// `tile`, the tiles' parts numbered in tile order; every wave finds its
-// item's tile with a prefix sum of the tiles' part counts over the lanes.
+// heads, work items of pa_item).
 template <int GQA>
 __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *__restrict__ Q,
                                                          const unsigned char *__restrict__ F, uint32_t c_lo,
@@ -917,36 +779,8 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
     const uint32_t kvh = blockIdx.x;
     // the work item's query tile and key part
     const PaGeom geo{(uint32_t)TQ, n_tok, num_prev, window, maxparts};
-    const uint32_t ntiles = (n_tok + TQ - 1) / TQ;
-    uint32_t tile = 0, part = 0, nparts = 1;
-    {
-        const uint32_t it = blockIdx.y;
-        uint32_t base = 0;
-        for (uint32_t t0 = 0; t0 < ntiles; t0 += 64) {
-            const uint32_t t = t0 + lane;
-            const uint32_t np = t < ntiles ? pa_parts(geo, t) : 0u;
-            uint32_t incl = np;                                    // inclusive prefix sum over the lanes
-#pragma unroll
-            for (int d = 1; d < 64; d *= 2) {
-                const uint32_t v = (uint32_t)__shfl_up((int)incl, d, 64);
-                incl += lane >= d ? v : 0u;
-            }
-            const uint32_t total = (uint32_t)__shfl((int)incl, 63, 64);
-            if (it < base + total) {
-                const uint32_t r = it - base;
-                const uint64_t hit = __ballot(r < incl && r >= incl - np);
-                const int L = __builtin_ctzll(hit);
-                tile = t0 + L;
-                nparts = (uint32_t)__shfl((int)np, L, 64);
-                part = r - ((uint32_t)__shfl((int)incl, L, 64) - nparts);
-                break;
-            }
-            base += total;
-        }
-        tile = __builtin_amdgcn_readfirstlane(tile);
-        part = __builtin_amdgcn_readfirstlane(part);
-        nparts = __builtin_amdgcn_readfirstlane(nparts);
-    }
+    uint32_t tile, part, nparts;
+    pa_item(geo, blockIdx.y, lane, tile, part, nparts);
     // this lane's query: column c of the wave's 16 rows
     const int qi = wave * 16 + c;
     const uint32_t tq = tile * TQ + qi / GQA, head = kvh * GQA + qi % GQA;
@@ -1152,12 +986,225 @@ __global__ __launch_bounds__(256) void k_prefill_attn_merge(const float *__restr
 #pragma unroll
     for (uint32_t p = 0; p < kPaParts; ++p) {
         if (p >= nparts) break;
-        const float a = mp[p] == -INFINITY ? 0.0f : __expf(mp[p] - mx);
+        const float a = mp[p] == -INFINITY ? 0.0f : expf(mp[p] - mx);
         t += v[p] * a;
         den += lp[p] * a;
     }
     const uint32_t width = num_q_heads * D;
     store_out4(out, outb, ntt, width, (uint32_t)(i / width), (uint32_t)(i % width), t * (1.0f / (den + 1e-9f)));
+}
+
+// ---------------------------------------------------------------------
+// Prefill attention on the matrix cores, head_dim 512, in fp32.
+//
+// A workgroup takes 16 query rows (16 / GQA tokens x the GQA heads of one KV
+// head) against the key list in steps of 16 keys with an online softmax;
+// both products run on v_mfma_f32_16x16x4_f32, so operands, products and sums
+// stay fp32 (head_dim 256's bf16 parts carry 6e-6 of the result, this kernel
+// and the per-token one it replaces 3e-7).  What bounds it: the fp32 matrix
+// rate (132 TFLOP/s in a large product on this card), of which the steps'
+// exchange and softmax leave about half.
+//  * Four waves take a quarter of the head (128 dims) each, of the scores'
+//    sum and of the output, so no K or V element is read by two waves and
+//    none needs LDS; the quarters of a step's scores meet in LDS (one barrier
+//    a step, two buffers) and every wave adds them in the same order.
+//  * S^T = K Q^T with the dims in the order that lane (key, g) loads them (a
+//    16-byte load holds its operand of four MFMAs); S^T's accumulator has
+//    keys 4g + i in lane group g, which is the B operand of step i of
+//    O^T = V^T P^T when lane group g supplies V rows 4g + i, and output row m
+//    of tile (b, e) is dim 64 b + 4 m + e, so a lane's 16-byte load of a V
+//    row feeds four tiles: probabilities and V stay in registers.
+//  * K of the next step is requested once this step's scores are summed, V
+//    once its products are done.
+// Keys that a query does not see have probability 0; where V holds a NaN or
+// an infinity among such keys, the step is multiplied token by token with
+// those rows left out (0 x Inf would reach the tokens before them).
+// Measured, 16 query / 4 KV heads, against one workgroup per token reading
+// every row: 200 tokens after 411 76 against 541 us, 1024 after 600 0.51
+// against 4.8 ms, 1 after 611 27 against 158 us.  Two query tiles per
+// workgroup (one wave per SIMD): 62 against 73 TFLOP/s on the largest.
+constexpr int kPa5Step = 16;              // keys per step
+template <int GQA>
+__global__ __launch_bounds__(256) void k_prefill_attn_d512(const float *__restrict__ Q, const float *__restrict__ Kc,
+                                                           const float *__restrict__ Vc,
+                                                           const uint32_t *__restrict__ slots, uint32_t num_prev,
+                                                           uint32_t n_tok, uint32_t num_q_heads, uint32_t kv_dim,
+                                                           float scale, uint32_t window, float *__restrict__ out,
+                                                           __bf16 *__restrict__ outb, float *__restrict__ ws,
+                                                           uint32_t maxparts, uint32_t ntt) {
+    constexpr uint32_t D = 512, TQ = 16 / GQA;
+    __shared__ f4 sbuf[2][4][64];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t g = lane >> 4, c = lane & 15;
+    const uint32_t kvh = blockIdx.x, n_keys = num_prev + n_tok;
+    const PaGeom geo{TQ, n_tok, num_prev, window, maxparts};
+    uint32_t tile, part, nparts;
+    pa_item(geo, blockIdx.y, lane, tile, part, nparts);
+    uint32_t cf, ce;
+    pa_chunks(geo, tile, cf, ce);
+    const uint32_t per = (ce - cf + nparts - 1) / nparts;
+    const uint32_t c_begin = min(ce, cf + part * per), c_stop = min(ce, c_begin + per);
+    // keys [k_begin, k_stop) of this part
+    const uint32_t t_last = min(tile * TQ + TQ, n_tok) - 1;
+    const uint32_t k_begin = c_begin * kPaNK, k_stop = min(c_stop * kPaNK, num_prev + t_last + 1);
+    auto seen_from = [&](uint32_t t) { return (window > 0 && num_prev + t + 1 > window) ? num_prev + t + 1 - window : 0; };
+    const uint32_t S_first = num_prev + tile * TQ + 1, start_last = seen_from(t_last);
+
+    // this lane's query: row c of the tile
+    const uint32_t tq = tile * TQ + c / GQA, tqc = min(tq, n_tok - 1), head = kvh * GQA + c % GQA;
+    const uint32_t Sq = num_prev + tqc + 1, startq = seen_from(tqc);
+    const uint32_t d0 = 128 * wave;                    // this wave's dims
+    const float *Kb = Kc + (size_t)kvh * D + d0 + 4 * g, *Vb = Vc + (size_t)kvh * D + d0 + 4 * c;
+    auto slot_at = [&](uint32_t k0) { return slots[min(k0 + c, n_keys - 1)]; };
+    f4 kf[8], vf[4][2];
+    auto load_k = [&](uint32_t slot) {
+        const float *p = Kb + (size_t)slot * kv_dim;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) kf[j] = *(const f4 *)(p + 16 * j);
+    };
+    auto load_v = [&](uint32_t slot) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float *p = Vb + (size_t)(uint32_t)__shfl((int)slot, 4 * g + i, 64) * kv_dim;
+            vf[i][0] = *(const f4 *)p;
+            vf[i][1] = *(const f4 *)(p + 64);
+        }
+    };
+    // (a part without keys runs no step; its loads read the last key's row)
+    const uint32_t slot = slot_at(k_begin);
+    uint32_t slot_n = slot_at(k_begin + kPa5Step);
+    load_k(slot);
+    load_v(slot);
+    f4 q[8];
+    {
+        const float *qr = Q + ((size_t)tqc * num_q_heads + head) * D + d0 + 4 * g;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = *(const f4 *)(qr + 16 * j);
+    }
+    f4 o[2][4];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[b][e] = f4{0, 0, 0, 0};
+    float m = -1e9f, l = 0.0f;
+    int buf = 0;
+    for (uint32_t k0 = k_begin; k0 < k_stop; k0 += kPa5Step, buf ^= 1) {
+        f4 sa[4];                                      // four shorter sums of the 128 dims, added in pairs
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sa[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], q[j][e], j == 0 ? f4{0, 0, 0, 0} : sa[e], 0, 0,
+                                                             0);
+        load_k(slot_n);
+        const uint32_t slot_2 = slot_at(k0 + 2 * kPa5Step);
+        sbuf[buf][wave][lane] = (sa[0] + sa[1]) + (sa[2] + sa[3]);
+        wait_vm_lgkm0<63>();                           // this wave's quarter is in LDS (loads stay in flight)
+        bare_barrier();                                // ... every wave's; the other buffer's reads are done
+        const f4 s = (sbuf[buf][0][lane] + sbuf[buf][1][lane]) + (sbuf[buf][2][lane] + sbuf[buf][3][lane]);
+        float p[4], mx = m, ps = 0.0f;
+        bool ok[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t kp = k0 + 4 * g + i;
+            ok[i] = kp >= startq && kp < Sq;
+            p[i] = s[i] * scale;
+            if (ok[i]) mx = fmaxf(mx, p[i]);
+        }
+        mx = rows4_max(mx);
+        const float alpha = expf(m - mx);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            p[i] = ok[i] ? expf(p[i] - mx) : 0.0f;
+            ps += p[i];
+        }
+        l = l * alpha + rows4_sum(ps);
+        m = mx;
+        bool split = false;
+        if (k0 + kPa5Step > S_first || k0 < start_last) {  // some query does not see some key of this step
+            float z = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) z = fmaf(vf[i][b][e], 0.0f, z);
+            split = __ballot(z != 0.0f) != 0;              // NaN: V holds a non-finite value
+        }
+        // The step's 16 keys are summed from zero, then added: a running sum
+        // over all keys in the accumulator would round four times as often
+        // (6.3e-7 against 3.1e-7 of the result over 1600 keys).
+        if (!split) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                f4 t[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        t[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][b][e], p[i], i == 0 ? f4{0, 0, 0, 0} : t[e],
+                                                                    0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[b][e] = o[b][e] * alpha + t[e];
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[b][e] *= alpha;
+            for (uint32_t tk = 0; tk < TQ; ++tk) {
+                const uint32_t tt = min(tile * TQ + tk, n_tok - 1), St = num_prev + tt + 1, st = seen_from(tt);
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        f4 t = f4{0, 0, 0, 0};         // (other tokens' columns may hold 0 x Inf: dropped)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t kp = k0 + 4 * g + i;
+                            t = __builtin_amdgcn_mfma_f32_16x16x4f32(kp >= st && kp < St ? vf[i][b][e] : 0.0f, p[i], t,
+                                                                     0, 0, 0);
+                        }
+                        if (c / GQA == tk) o[b][e] += t;
+                    }
+            }
+        }
+        load_v(slot_n);
+        slot_n = slot_2;
+    }
+    if (tq >= n_tok) return;
+    const size_t nrow = (size_t)n_tok * num_q_heads, row = (size_t)tq * num_q_heads + head;
+    const float inv = 1.0f / (l + 1e-9f);
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const f4 v = f4{o[b][0][i], o[b][1][i], o[b][2][i], o[b][3][i]};
+            const uint32_t d = d0 + 64 * b + 16 * g + 4 * i;
+            if (nparts > 1)                            // unnormalised, as k_prefill_attn_mf leaves its parts
+                *(f4 *)(ws + (part * nrow + row) * D + d) = v;
+            else
+                store_out4(out, outb, ntt, num_q_heads * D, tq, head * D + d, v * inv);
+        }
+    if (nparts > 1 && wave == 0 && g == 0) {
+        float *ml = ws + maxparts * nrow * D + 2 * (part * nrow + row);
+        ml[0] = m;
+        ml[1] = l;
+    }
+}
+
+// Parts of the key list at head_dim 512: until there are 400 workgroups (a
+// step's exchange leaves a lone workgroup's matrix cores idle; 200 tokens
+// after 411 on 4 KV heads: 2 parts 76, 4 parts 81 us), and so that a part's
+// sums run over about 1024 keys at most (their rounding grows with the
+// length: over 1600 keys 3.1e-7 in one part, 3.0e-7 in the per-token kernel).
+static uint32_t pa5_parts(uint32_t n_tok, uint32_t n_keys, uint32_t gqa, uint32_t num_kv) {
+    const uint32_t wgs = (n_tok * gqa + 15) / 16 * num_kv;
+    uint32_t parts = 1;
+    while (parts < kPaParts && (wgs * parts < 400 || n_keys > 1024 * parts)) parts *= 2;
+    return parts;
 }
 
 static int launch_decode_impl(chn_ctx *ctx, const float *q, float *kc, float *vc, const uint32_t *slots,
@@ -1239,6 +1286,25 @@ bool prefill_frags_fusable(uint32_t num_prev, uint32_t head_dim, uint32_t gqa) {
     return head_dim == 256 && (gqa == 1 || gqa == 2 || gqa == 4 || gqa == 8) && num_prev % kPaNK == 0;
 }
 
+// Work items per KV head; returns whether any tile is cut into parts.
+static bool pa_items(const PaGeom &geo, uint32_t &items) {
+    bool split = false;
+    items = 0;
+    for (uint32_t t = 0; t < (geo.n_tok + geo.TQ - 1) / geo.TQ; ++t) {
+        const uint32_t np = pa_parts(geo, t);
+        items += np;
+        split |= np > 1;
+    }
+    return split;
+}
+
+static void launch_pa_merge(hipStream_t st, const float *ws, const PaGeom &geo, uint32_t num_q_heads, uint32_t D,
+                            float *out, __bf16 *outb, uint32_t ntt) {
+    const size_t nrow = (size_t)geo.n_tok * num_q_heads;
+    k_prefill_attn_merge<<<(unsigned)((nrow * D / 4 + 255) / 256), 256, 0, st>>>(ws, geo, num_q_heads, nrow, D, out,
+                                                                                 outb, ntt);
+}
+
 int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const float *vc, const uint32_t *slots,
                         uint32_t n_tok, uint32_t num_prev, uint32_t num_q_heads, uint32_t head_dim, uint32_t kv_dim,
                         uint32_t gqa, float scale, uint32_t window, float *out, __bf16 *outb, float *ws,
@@ -1257,19 +1323,14 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
             k_prefill_frags<<<dim3(num_kv, c_pre - c_lo, 2), 256, 0, st>>>(kc, vc, slots, n_keys, c_lo, nfch,
                                                                          kv_dim, frag);
         const uint32_t tq = 16 * kPaWaves / gqa;
-        const uint32_t tiles = (n_tok + tq - 1) / tq;
         // Causal tiles differ in length (the last one walks every key): each
         // tile's chunks are cut into parts of about kPaPartChunks chunks (at
         // most kPaParts), so the longest walk is about that long and the
         // short tiles run whole (512 tokens: 16 tiles of 1..16 chunks -> 40
         // parts of at most 4 chunks per KV head).
         const PaGeom geo{tq, n_tok, num_prev, window, ws ? kPaParts : 1u};
-        uint32_t items = 0, split_tiles = 0;
-        for (uint32_t t = 0; t < tiles; ++t) {
-            const uint32_t np = pa_parts(geo, t);
-            items += np;
-            split_tiles += np > 1 ? 1u : 0u;
-        }
+        uint32_t items = 0;
+        const bool split = pa_items(geo, items);
         const dim3 mgrid(num_q_heads / gqa, items);
 #define CHN_PATTN_MF(G)                                                                                  \
     k_prefill_attn_mf<G><<<mgrid, 64 * kPaWaves, 0, st>>>(q, frag, c_lo, nfch, num_prev, n_tok, num_q_heads, scale, \
@@ -1281,37 +1342,26 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
         default: CHN_PATTN_MF(8); break;
         }
 #undef CHN_PATTN_MF
-        if (split_tiles) {
-            const size_t nrow = (size_t)n_tok * num_q_heads, nq4 = nrow * head_dim / 4;
-            k_prefill_attn_merge<<<(unsigned)((nq4 + 255) / 256), 256, 0, st>>>(ws, geo, num_q_heads, nrow, head_dim,
-                                                                                  out, outb, ntt);
-        }
+        if (split) launch_pa_merge(st, ws, geo, num_q_heads, head_dim, out, outb, ntt);
         return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
     }
-    dim3 grid(n_tok, num_q_heads / gqa);
-#define CHN_PATTN(DV, G) \
-    k_prefill_attn<DV, G><<<grid, 256, 0, st>>>(q, kc, vc, slots, num_prev, num_q_heads, kv_dim, scale, window, out, \
-                                                outb, ntt)
-    if (head_dim == 256) {
-        switch (gqa) {
-        case 1: CHN_PATTN(1, 1); break;
-        case 2: CHN_PATTN(1, 2); break;
-        case 4: CHN_PATTN(1, 4); break;
-        case 8: CHN_PATTN(1, 8); break;
-        default: return CHN_E_UNSUPPORTED;
-        }
-    } else if (head_dim == 512) {
-        switch (gqa) {
-        case 1: CHN_PATTN(2, 1); break;
-        case 2: CHN_PATTN(2, 2); break;
-        case 4: CHN_PATTN(2, 4); break;
-        default: return CHN_E_UNSUPPORTED;
-        }
-    } else {
-        return CHN_E_UNSUPPORTED;
+    if (head_dim == 512 && (gqa == 1 || gqa == 2 || gqa == 4)) {
+        const uint32_t num_kv = num_q_heads / gqa;
+        const PaGeom geo{16 / gqa, n_tok, num_prev, window, ws ? pa5_parts(n_tok, num_prev + n_tok, gqa, num_kv) : 1u};
+        uint32_t items = 0;
+        const bool split = pa_items(geo, items);
+        const dim3 grid(num_kv, items);
+#define CHN_PATTN5(G)                                                                                              \
+    k_prefill_attn_d512<G><<<grid, 256, 0, st>>>(q, kc, vc, slots, num_prev, n_tok, num_q_heads, kv_dim, scale, \
+                                                 window, out, outb, ws, geo.maxparts, ntt)
+        if (gqa == 1) CHN_PATTN5(1);
+        else if (gqa == 2) CHN_PATTN5(2);
+        else CHN_PATTN5(4);
+#undef CHN_PATTN5
+        if (split) launch_pa_merge(st, ws, geo, num_q_heads, head_dim, out, outb, ntt);
+        return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
     }
-#undef CHN_PATTN
-    return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
+    return CHN_E_UNSUPPORTED;
 }
 
 // ---------------------------------------------------------------------
