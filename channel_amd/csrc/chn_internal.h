@@ -259,19 +259,23 @@ int launch_topk64(hipStream_t st, const float *logits, uint32_t V, uint32_t *ids
 int launch_embed(hipStream_t st, const uint16_t *table, const uint32_t *tokens, uint32_t n, uint32_t H, float scale,
                  float *x);
 int launch_quantize(hipStream_t st, int q8, const uint16_t *src, uint32_t *dst, uint64_t nblk);
-// Contractions of at most kFewTokens tokens run on gemm_q4_few.hip, whose
-// bf16 activations lie in operand order (xb_at); larger ones read them row
-// by row.  At 128 tokens the few-token kernels lead or tie on every 12B shape
-// (gate/up 77 against 118 us, down 51 / 57, q/k/v 20 / 31, o_proj 18 / 20);
-// at 192 they trail on down (76 / 59) and o_proj (26 / 22).
-constexpr uint32_t kFewTokens = 128;
-inline bool few_tokens(uint32_t n_tok) { return n_tok <= kFewTokens; }
+// Contractions of few tokens run on gemm_q4_few.hip, whose bf16 activations
+// lie in operand order (xb_at); larger ones read them row by row.  The
+// limits are where the two meet at 12B dims (both with their bf16 pass, us):
+// gate/up 48 tokens 38 / 44, 64 tokens 43 / 44, 80 tokens 51 / 46; long K
+// (down) 48 tokens 31 / 40, 65 tokens 50 / 40; q/k/v 128 tokens 27 / 36.
+constexpr uint32_t kFewTokens = 128, kFewTokensWide = 64;
+inline bool few_tokens(uint32_t n_tok, int nmat, uint32_t K) {
+    return n_tok <= (nmat == 2 || K >= 8192 ? kFewTokensWide : kFewTokens);
+}
 inline uint32_t xb_tiles(uint32_t n_tok) { return (n_tok + 15) / 16; }
-// Tile count to pass as xb_at's ntt for a contraction of n_tok tokens.
-inline uint32_t xb_layout(uint32_t n_tok) { return few_tokens(n_tok) ? xb_tiles(n_tok) : 0u; }
+// xb_at's ntt for the activations of a contraction of n_tok tokens.
+inline uint32_t xb_layout(uint32_t n_tok, int nmat, uint32_t K) {
+    return few_tokens(n_tok, nmat, K) ? xb_tiles(n_tok) : 0u;
+}
 // Elements of the bf16 activation buffer of n_tok tokens of width K.
-inline size_t xb_elems(uint32_t n_tok, uint32_t K) {
-    return few_tokens(n_tok) ? (size_t)xb_tiles(n_tok) * 16 * ((K + 255) / 256) * 256 : (size_t)n_tok * K;
+inline size_t xb_elems(uint32_t n_tok, uint32_t K, int nmat) {
+    return few_tokens(n_tok, nmat, K) ? (size_t)xb_tiles(n_tok) * 16 * ((K + 255) / 256) * 256 : (size_t)n_tok * K;
 }
 // Element (token t, k) of bf16 activations of `width` columns: row-major
 // when ntt is 0, else operand order of k_q4gemm_few over ntt tiles of 16
@@ -286,19 +290,19 @@ __host__ __device__ inline size_t xb_at(uint32_t ntt, uint32_t width, uint32_t t
 int launch_to_bf16_few(hipStream_t st, const float *X, __bf16 *xb, uint32_t n_tok, uint32_t K);
 // nseg matrices over the same activations (nmat 1), or gate W[0] and up W1
 // (nmat 2).  Yb (nmat 2): the result as bf16 instead of Y[0], in xb_at order
-// when yb_frag, else row-major.
+// for yb_ntt.
 int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1, float *const *Y,
                       const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked,
-                      __bf16 *Yb = nullptr, bool yb_frag = false);
+                      __bf16 *Yb = nullptr, uint32_t yb_ntt = 0);
 // W0/W1 in the reference Q4 layout, or in Q4R with repacked.  X (fp32) is
 // converted into xb (xb_elems); with X == NULL, xb already holds the bf16
-// activations, in xb_at order for xb_layout(n_tok).
+// activations, in xb_at order for xb_layout(n_tok, nmat, K).
 // Yb (two-matrix form only): the result goes to Yb as bf16 instead of Y,
-// in the next contraction's order when X == NULL, else row-major.
+// in the order of a one-matrix contraction when X == NULL, else row-major.
 // po (single matrix): a shape that splits K may store its partial sums to
-// Y + p * po->stride, p < po->max_parts (1, 2 or 4), with plain stores
-// instead of clearing Y and adding into it; po->parts tells how many it
-// wrote (their sum, in index order, is the result).
+// Y + p * po->stride, p < po->max_parts (1, 2 or 4), instead of summing them
+// itself; po->parts tells how many it wrote (their sum, in index order, is
+// the result).
 struct PartialOut {
     size_t stride = 0;         // elements between partial outputs
     uint32_t max_parts = 1;

@@ -262,7 +262,7 @@ static void launch_few_shape(hipStream_t st, FewArgs &a, int nseg) {
 
 int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1, float *const *Y,
                       const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked, __bf16 *Yb,
-                      bool yb_frag) {
+                      uint32_t yb_ntt) {
     FewArgs a{};
     a.X = xb;
     for (int s = 0; s < nseg; ++s) {
@@ -275,7 +275,7 @@ int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const 
     a.n_tok = n_tok;
     a.K = K;
     a.ntt = xb_tiles(n_tok);
-    a.yb_ntt = yb_frag ? a.ntt : 0;
+    a.yb_ntt = yb_ntt;
     if (nmat == 2) {
         if (repacked) launch_few_shape<2, true>(st, a, nseg);
         else launch_few_shape<2, false>(st, a, nseg);
