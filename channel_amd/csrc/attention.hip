@@ -1365,7 +1365,7 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
 }
 
 // ---------------------------------------------------------------------
-// qkv_rope: one 64-lane workgroup per head.
+// qkv_rope and batch_qkv_rope.
 // ---------------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -1373,113 +1373,141 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// RMSNorm * w, then RoPE on pairs (d, d + rot/2) at `clock`, suffix past
-// rot copied (shaders/qkv_rope.wgsl:42-91).
-__device__ void norm_rope_head(const float *__restrict__ in, const float *__restrict__ w, float *__restrict__ out,
-                               uint32_t D, uint32_t rot, float theta, float eps, uint32_t clock, float *buf,
-                               const float2 *__restrict__ cs_tab = nullptr) {
-    const int lane = threadIdx.x;
-    float ss = 0.0f;
-    for (uint32_t d = lane; d < D; d += 64) ss += in[d] * in[d];
-    ss = wave_sum(ss);
-    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-    for (uint32_t d = lane; d < D; d += 64) buf[d] = (in[d] * inv) * w[d];
-    __syncthreads();
-    const uint32_t half = rot / 2;
-    for (uint32_t d = lane; d < half; d += 64) {
-        const float v0 = buf[d], v1 = buf[d + half];
-        float c, s;
-        if (cs_tab) {
-            const float2 t = cs_tab[d];
-            c = t.x;
-            s = t.y;
-        } else {
-            const float fe = (2.0f * (float)d) / (float)rot;
-            const float freq = 1.0f / powf(theta, fe);
-            const float ang = (float)clock * freq;
-            c = cosf(ang);
-            s = sinf(ang);
+struct QkvRope {
+    const float *q_in, *k_in, *v_in, *qw, *kw;   // v_in: k_in where V is the raw K
+    float *q_out, *kc, *vc;
+    const uint32_t *step;                        // decode: {clock, slot} of the one token, or NULL
+    const uint32_t *slots;                       // batch: token t's slot is slots[slot_offset + t], its clock start_clock + t
+    uint32_t slot_offset, start_clock, num_q, num_kv, D, rot;
+    float theta, eps;
+    const float2 *tab;                           // (cos, sin) per token and pair (launch_rope_tab_batch), or NULL
+};
+
+// RMSNorm * w, then RoPE on pairs (d, d + rot/2), suffix past rot copied, for
+// the query and key heads, unit RMSNorm for V (shaders/qkv_rope.wgsl:42-91,
+// shaders/batch_qkv_rope.wgsl); any head_dim up to 64 * DPL, any even rot, any
+// alignment.
+//
+// What bounds it: the angles and one chain of dependent steps, not the rows
+// (300 tokens of 16 + 2 x 8 heads of 256: 20 MB, 4 us).  A power, a sine and a
+// cosine per pair were evaluated once per head by the wave that rotates it;
+// here a workgroup takes 4 * HPW rows (a wave takes HPW of them, V rows like
+// query and key rows) of ONE token, evaluates that token's angles once, one
+// per thread, while its rows are on their way, and hands them round in LDS.
+template <int DPL, int HPW>
+__global__ __launch_bounds__(256) void k_qkv_rope(QkvRope a) {
+    __shared__ float2 cs[256];
+    __shared__ float buf[4][64 * DPL];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t t = blockIdx.y, D = a.D, half = a.rot / 2;
+    const uint32_t nrow = a.num_q + 2 * a.num_kv, row0 = (blockIdx.x * 4 + wave) * HPW;
+    const size_t q_dim = (size_t)a.num_q * D, kv_dim = (size_t)a.num_kv * D;
+
+    // the rows (values past D load the last one and are left out below)
+    float v[HPW][DPL], w[HPW][DPL];
+#pragma unroll
+    for (int i = 0; i < HPW; ++i) {
+        const uint32_t row = min(row0 + i, nrow - 1);
+        const bool q = row < a.num_q, k = !q && row < a.num_q + a.num_kv;
+        const uint32_t h = q ? row : (k ? row - a.num_q : row - a.num_q - a.num_kv);
+        const float *in = (q ? a.q_in + t * q_dim : (k ? a.k_in : a.v_in) + t * kv_dim) + (size_t)h * D;
+        const float *nw = q ? a.qw : a.kw;
+#pragma unroll
+        for (int j = 0; j < DPL; ++j) {
+            const uint32_t d = min(lane + 64u * j, D - 1);
+            v[i][j] = in[d];
+            w[i][j] = nw[d];
         }
-        out[d] = v0 * c - v1 * s;
-        out[d + half] = v0 * s + v1 * c;
     }
-    for (uint32_t d = rot + lane; d < D; d += 64) out[d] = buf[d];
+    const uint32_t clock = a.step ? a.step[0] : a.start_clock + t;
+    const uint32_t slot = a.step ? a.step[1] : a.slots[a.slot_offset + t];
+    if ((uint32_t)tid < half) {
+        if (a.tab) {
+            cs[tid] = a.tab[(size_t)t * half + tid];
+        } else {
+            const float fe = (2.0f * (float)tid) / (float)a.rot;
+            const float freq = 1.0f / powf(a.theta, fe);
+            const float ang = (float)clock * freq;
+            float sn, c;
+            sincosf(ang, &sn, &c);
+            cs[tid] = float2{c, sn};
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < HPW; ++i) {
+        const uint32_t row = row0 + i;
+        if (row >= nrow) return;                       // a whole wave; no barrier follows
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < DPL; ++j)
+            if (lane + 64u * j < D) ss += v[i][j] * v[i][j];
+        ss = wave_sum(ss);
+        const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
+        if (row >= a.num_q + a.num_kv) {
+            float *o = a.vc + (size_t)slot * kv_dim + (size_t)(row - a.num_q - a.num_kv) * D;
+#pragma unroll
+            for (int j = 0; j < DPL; ++j)
+                if (lane + 64u * j < D) o[lane + 64 * j] = v[i][j] * inv;
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < DPL; ++j) {
+            v[i][j] = (v[i][j] * inv) * w[i][j];
+            buf[wave][lane + 64 * j] = v[i][j];
+        }
+        // the wave reads only what it wrote itself
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float *o = row < a.num_q ? a.q_out + t * q_dim + (size_t)row * D
+                                 : a.kc + (size_t)slot * kv_dim + (size_t)(row - a.num_q) * D;
+#pragma unroll
+        for (int j = 0; j < DPL; ++j) {
+            const uint32_t d = lane + 64 * j;
+            if (d >= D) continue;
+            float r = v[i][j];
+            if (d < half) {
+                r = r * cs[d].x - buf[wave][d + half] * cs[d].y;
+            } else if (d < a.rot) {
+                r = buf[wave][d - half] * cs[d - half].y + r * cs[d - half].x;
+            }
+            o[d] = r;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();               // before the next row overwrites buf
+    }
 }
 
-__global__ __launch_bounds__(64) void k_qkv_rope(const float *__restrict__ q_in, const float *__restrict__ k_in,
-                                                 const float *__restrict__ v_in, const float *__restrict__ qw,
-                                                 const float *__restrict__ kw, float *__restrict__ q_out,
-                                                 float *__restrict__ k_cache, float *__restrict__ v_cache,
-                                                 const uint32_t *__restrict__ step, uint32_t num_q,
-                                                 uint32_t num_kv, uint32_t D, uint32_t rot, int k_eq_v,
-                                                 float theta, float eps) {
-    __shared__ float buf[512];
-    const uint32_t head = blockIdx.x;
-    const uint32_t clock = step[0], slot = step[1];
-    if (head < num_q) {
-        norm_rope_head(q_in + (size_t)head * D, qw, q_out + (size_t)head * D, D, rot, theta, eps, clock, buf);
-        return;
-    }
-    const uint32_t h = head - num_q;
-    if (h >= num_kv) return;
-    const size_t kv_dim = (size_t)num_kv * D;
-    const float *k = k_in + (size_t)h * D;
-    const float *v = k_eq_v ? k : v_in + (size_t)h * D;
-    norm_rope_head(k, kw, k_cache + (size_t)slot * kv_dim + (size_t)h * D, D, rot, theta, eps, clock, buf);
-    // V: unit RMSNorm (no weight)
-    const int lane = threadIdx.x;
-    float ss = 0.0f;
-    for (uint32_t d = lane; d < D; d += 64) ss += v[d] * v[d];
-    ss = wave_sum(ss);
-    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-    float *vo = v_cache + (size_t)slot * kv_dim + (size_t)h * D;
-    for (uint32_t d = lane; d < D; d += 64) vo[d] = v[d] * inv;
+template <int DPL, int HPW>
+static void launch_rope_rows(hipStream_t st, const QkvRope &a, uint32_t n_tok) {
+    const uint32_t nrow = a.num_q + 2 * a.num_kv, per = 4 * HPW;
+    k_qkv_rope<DPL, HPW><<<dim3((nrow + per - 1) / per, n_tok), 256, 0, st>>>(a);
 }
 
-// batch_qkv_rope (shaders/batch_qkv_rope.wgsl): token t uses clock
-// start_clock + t and writes its K/V at slot slots[slot_offset + t].
-__global__ __launch_bounds__(64) void k_batch_qkv_rope(const float *__restrict__ q_in, const float *__restrict__ k_in,
-                                                       const float *__restrict__ v_in, const float *__restrict__ qw,
-                                                       const float *__restrict__ kw, float *__restrict__ q_out,
-                                                       float *__restrict__ k_cache, float *__restrict__ v_cache,
-                                                       const uint32_t *__restrict__ slots, uint32_t slot_offset,
-                                                       uint32_t start_clock, uint32_t num_q, uint32_t num_kv,
-                                                       uint32_t D, uint32_t rot, int k_eq_v, float theta, float eps,
-                                                       const float2 *__restrict__ tab) {
-    __shared__ float buf[512];
-    const uint32_t head = blockIdx.x, t = blockIdx.y;
-    const uint32_t clock = start_clock + t, slot = slots[slot_offset + t];
-    const size_t q_dim = (size_t)num_q * D, kv_dim = (size_t)num_kv * D;
-    const float2 *cs = tab ? tab + (size_t)t * (rot / 2) : nullptr;
-    if (head < num_q) {
-        norm_rope_head(q_in + t * q_dim + (size_t)head * D, qw, q_out + t * q_dim + (size_t)head * D, D, rot, theta,
-                       eps, clock, buf, cs);
-        return;
-    }
-    const uint32_t h = head - num_q;
-    if (h >= num_kv) return;
-    const float *k = k_in + t * kv_dim + (size_t)h * D;
-    const float *v = k_eq_v ? k : v_in + t * kv_dim + (size_t)h * D;
-    norm_rope_head(k, kw, k_cache + (size_t)slot * kv_dim + (size_t)h * D, D, rot, theta, eps, clock, buf, cs);
-    const int lane = threadIdx.x;
-    float ss = 0.0f;
-    for (uint32_t d = lane; d < D; d += 64) ss += v[d] * v[d];
-    ss = wave_sum(ss);
-    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-    float *vo = v_cache + (size_t)slot * kv_dim + (size_t)h * D;
-    for (uint32_t d = lane; d < D; d += 64) vo[d] = v[d] * inv;
+// Two rows per wave where the launch has kRopeRows rows or more (16 + 2 x 8
+// heads of 256: 300 tokens 6.8 us against 7.6 with one, 1024 tokens 15.0
+// against 17.4), one below (one token 3.3 against 4.0, 128 tokens 4.8 against
+// 5.0: a second row only makes the chain longer) and for the wider heads (300
+// tokens 6.6 against 7.4).  Before, with angles per head: one token 5.2 us,
+// 128 tokens 7.2, 300 tokens 11.8, 1024 tokens 30.8.
+constexpr size_t kRopeRows = 8192;
+static int launch_rope_any(hipStream_t st, const QkvRope &a, uint32_t n_tok) {
+    if (a.D > 256) launch_rope_rows<8, 1>(st, a, n_tok);
+    else if ((size_t)n_tok * (a.num_q + 2 * a.num_kv) >= kRopeRows) launch_rope_rows<4, 2>(st, a, n_tok);
+    else launch_rope_rows<4, 1>(st, a, n_tok);
+    return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
 }
 
 int launch_qkv_rope(hipStream_t st, const float *q_in, const float *k_in, const float *v_in, const float *qw,
                     const float *kw, float *q_out, float *kc, float *vc, const uint32_t *step, uint32_t num_q,
                     uint32_t num_kv, uint32_t D, uint32_t rot, int k_eq_v, float theta, float eps) {
-    k_qkv_rope<<<num_q + num_kv, 64, 0, st>>>(q_in, k_in, v_in, qw, kw, q_out, kc, vc, step, num_q, num_kv, D, rot,
-                                              k_eq_v, theta, eps);
-    return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
+    return launch_rope_any(st, QkvRope{q_in, k_in, k_eq_v ? k_in : v_in, qw, kw, q_out, kc, vc, step, nullptr, 0, 0,
+                                       num_q, num_kv, D, rot, theta, eps, nullptr}, 1);
 }
 
-// The same with four heads per workgroup, one per wave, for D a multiple of
-// 256 and the angle table given: lane l holds dims 4 l + 256 j .. +3 (one
+// Four heads per workgroup, one per wave, for D a multiple of 256 and the
+// angle table given: lane l holds dims 4 l + 256 j .. +3 (one
 // 16-byte access each), the norm reduces across the wave, and each wave
 // pairs (d, d + rot/2) through its own LDS row (a wave reads only what it
 // wrote, so no workgroup barrier is needed).
@@ -1742,10 +1770,8 @@ int launch_batch_qkv_rope(hipStream_t st, const float *q_in, const float *k_in, 
                                                         num_q, num_kv, rot, k_eq_v, eps, tab);
         return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
     }
-    dim3 grid(num_q + num_kv, n_tok);
-    k_batch_qkv_rope<<<grid, 64, 0, st>>>(q_in, k_in, v_in, qw, kw, q_out, kc, vc, slots, slot_offset, start_clock,
-                                          num_q, num_kv, D, rot, k_eq_v, theta, eps, tab);
-    return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
+    return launch_rope_any(st, QkvRope{q_in, k_in, k_eq_v ? k_in : v_in, qw, kw, q_out, kc, vc, nullptr, slots,
+                                       slot_offset, start_clock, num_q, num_kv, D, rot, theta, eps, tab}, n_tok);
 }
 
 // (cos, sin) of (start_clock + t) * theta^(-2d / rot) for t < n_tok, d <
