@@ -19,6 +19,12 @@
 //    weight load of a wave asks for 16 whole 128-byte lines.  (Blocks g and
 //    4 + g, half lines per load: 28.0 against 23.5 us for gate/up at 8
 //    tokens; non-temporal loads of half lines, each line fetched twice: 31.)
+//  * What is left to bound it is instruction issue: a wave issues a VALU
+//    operation every 8 cycles at most, two waves of a SIMD one every 4.7, and
+//    waves wait to issue 46 % of their time, for memory 19 %.  Loads count
+//    too: the scales of a lane's two blocks (Q4R) come in one 4-byte load
+//    (two 2-byte loads: gate/up at 24 tokens 27.4 against 25.9 us a call, at
+//    64 tokens 43.2 against 40.8; down at 24 tokens 25.8 against 24.9).
 //  * The waves of a workgroup share its feature tiles and take every
 //    WK-th step, so together they read the rows front to back; their sums
 //    meet in LDS in wave order (results do not depend on timing).
@@ -41,6 +47,7 @@ typedef __bf16 fbf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 fbf16x2 __attribute__((ext_vector_type(2)));
 typedef float ff32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t fu32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
 
 struct FewArgs {
     const __bf16 *X;                   // activations in xb_at order, ntt token tiles
@@ -107,7 +114,7 @@ __global__ __launch_bounds__(64 * WK) void k_q4gemm_few(FewArgs a) {
 
     struct Wstep {
         fu32x4 q[NF][2];
-        uint32_t s[NF][2];
+        uint32_t s[NF][REP ? 1 : 2];                   // REP: the two blocks' scales in one word
     };
     struct Xhalf {
         fu32x4 x[NT][4];
@@ -118,13 +125,15 @@ __global__ __launch_bounds__(64 * WK) void k_q4gemm_few(FewArgs a) {
     auto load_w = [&](uint32_t i, Wstep &w) {
         const uint32_t b0 = 8 * step(i) + 2 * g;
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
+        for (int f = 0; f < NF; ++f) {
+            // the scales of blocks b0 and b0 + 1, or of the row's last two
+            // (the word before a row's scales is readable: codes or scales)
+            if (REP) w.s[f][0] = *(const u32_a2 *)(ws[f] + (ptrdiff_t)min((int)b0, (int)nb - 2) * 2);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const size_t b = min(b0 + h, nb - 1);
                 if (REP) {
                     w.q[f][h] = *(const fu32x4 *)(wq[f] + b * 16);
-                    w.s[f][h] = *(const uint16_t *)(ws[f] + b * 2);
                 } else {
                     const uint32_t *p = (const uint32_t *)(wq[f] + b * 20);
                     const u32x4_a4 v = *(const u32x4_a4 *)(p + 1);
@@ -132,6 +141,7 @@ __global__ __launch_bounds__(64 * WK) void k_q4gemm_few(FewArgs a) {
                     w.q[f][h] = fu32x4{v[0], v[1], v[2], v[3]};
                 }
             }
+        }
     };
     auto load_x = [&](uint32_t i, int h, Xhalf &x) {
         const __bf16 *p = xf + ((size_t)step(i) * 2 + h) * a.ntt * 2048;
@@ -147,9 +157,10 @@ __global__ __launch_bounds__(64 * WK) void k_q4gemm_few(FewArgs a) {
         for (int t = 0; t < NT; ++t) acc[f][t] = ff32x4{0, 0, 0, 0};
     const bool ragged = (nb & 7) != 0;                 // the last step has blocks past the row's end
     auto compute = [&](uint32_t i, int h, const Wstep &w, Xhalf &x) {
-        uint32_t ok = 0xffffffffu;
+        uint32_t ok = 0xffffffffu, sh = 16 * h;
         if (ragged) {                                  // those contribute exact zeros on both sides
             ok = opaque_mask(8 * step(i) + 2 * g + h < nb);
+            if (8 * step(i) + 2 * g + 1 >= nb) sh = 16;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -157,7 +168,7 @@ __global__ __launch_bounds__(64 * WK) void k_q4gemm_few(FewArgs a) {
         }
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
-            const float s16 = 16.0f * f16_lo_to_f32(w.s[f][h] & ok);
+            const float s16 = 16.0f * f16_lo_to_f32((REP ? w.s[f][0] >> sh : w.s[f][h]) & ok);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const fbf16x8 d = few_dequant(REP ? w.q[f][h][j] : w.q[f][h][j] ^ 0x88888888u, s16);
