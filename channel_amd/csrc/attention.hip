@@ -45,9 +45,10 @@ size_t attn_ws_bytes(uint32_t num_q_heads, uint32_t head_dim, uint32_t max_slots
 }
 
 // Prefill key split: a query tile's key chunks are cut into parts of about
-// kPaPartChunks chunks, at most kPaParts parts (one workgroup each), so the
-// causal tiles' walks come out about equally long; the workspace holds each
-// part's sums [n_tok][heads][D] and (max, denominator) pairs.
+// kPaPartChunks chunks or more (pa_part_chunks), at most kPaParts parts (one
+// workgroup each), so the causal tiles' walks come out about equally long;
+// the workspace holds each part's sums [n_tok][heads][D] and (max,
+// denominator) pairs.
 constexpr uint32_t kPaParts = 4;
 constexpr uint32_t kPaPartChunks = 4;
 // Waves per prefill attention workgroup, 16 query rows each: eight waves
@@ -708,7 +709,7 @@ __global__ __launch_bounds__(256) void k_prefill_frags(const float *__restrict__
 // token's window start to its last token's key) and the number of parts it
 // is cut into (maxparts = 1: none).
 struct PaGeom {
-    uint32_t TQ, n_tok, num_prev, window, maxparts;
+    uint32_t TQ, n_tok, num_prev, window, maxparts, pchunks;
 };
 __host__ __device__ inline void pa_chunks(const PaGeom &g, uint32_t tile, uint32_t &cf, uint32_t &ce) {
     const uint32_t t_first = tile * g.TQ;
@@ -721,7 +722,7 @@ __host__ __device__ inline void pa_chunks(const PaGeom &g, uint32_t tile, uint32
 __host__ __device__ inline uint32_t pa_parts(const PaGeom &g, uint32_t tile) {
     uint32_t cf, ce;
     pa_chunks(g, tile, cf, ce);
-    const uint32_t np = (ce - cf + kPaPartChunks - 1) / kPaPartChunks;
+    const uint32_t np = (ce - cf + g.pchunks - 1) / g.pchunks;
     return np < 1 ? 1 : (np > g.maxparts ? g.maxparts : np);
 }
 
@@ -769,7 +770,7 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
                                                          uint32_t nfch, uint32_t num_prev, uint32_t n_tok,
                                                          uint32_t num_q_heads, float scale, uint32_t window,
                                                          float *__restrict__ out, __bf16 *__restrict__ outb,
-                                                         float *__restrict__ ws, uint32_t maxparts, uint32_t ntt) {
+                                                         float *__restrict__ ws, uint32_t maxparts, uint32_t pchunks, uint32_t ntt) {
     constexpr int D = 256, NK = kPaNK, TQ = 16 * kPaWaves / GQA;
     __shared__ __attribute__((aligned(16))) unsigned char ring[2][kPaChunkBytes];   // two chunks in flight
 
@@ -778,7 +779,7 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
     const int g = lane >> 4, c = lane & 15;
     const uint32_t kvh = blockIdx.x;
     // the work item's query tile and key part
-    const PaGeom geo{(uint32_t)TQ, n_tok, num_prev, window, maxparts};
+    const PaGeom geo{(uint32_t)TQ, n_tok, num_prev, window, maxparts, pchunks};
     uint32_t tile, part, nparts;
     pa_item(geo, blockIdx.y, lane, tile, part, nparts);
     // this lane's query: column c of the wave's 16 rows
@@ -1039,7 +1040,7 @@ __global__ __launch_bounds__(256) void k_prefill_attn_d512(const float *__restri
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t g = lane >> 4, c = lane & 15;
     const uint32_t kvh = blockIdx.x, n_keys = num_prev + n_tok;
-    const PaGeom geo{TQ, n_tok, num_prev, window, maxparts};
+    const PaGeom geo{TQ, n_tok, num_prev, window, maxparts, kPaPartChunks};
     uint32_t tile, part, nparts;
     pa_item(geo, blockIdx.y, lane, tile, part, nparts);
     uint32_t cf, ce;
@@ -1298,6 +1299,46 @@ static bool pa_items(const PaGeom &geo, uint32_t &items) {
     return split;
 }
 
+// Chunks per part at head_dim 256, where a CU holds one workgroup.  Causal
+// tiles differ in length (the last one walks every key), so short parts even
+// the walks out (512 tokens: 16 tiles of 1..16 chunks in parts of at most 4),
+// but each costs its prologue (about 1.2 chunks: Q and the first chunk) and a
+// share of the merge, and what matters first is that the parts fill the 256
+// CUs in whole rounds.  The estimate of the walk in chunks -- the longest part
+// of a single round, the mean part times the rounds otherwise -- ranks the
+// lengths as they measured (16 heads on 8 KV heads, us, parts of 4 chunks and
+// as chosen): 768 tokens 59 / 41, 1024 tokens 70 / 55, 1024 tokens after 1500
+// with a window of 1024 97 / 81 (two parts per tile, one round of 256, instead
+// of four and two rounds), 512 tokens after 512 50 / 48; 512 tokens 35 with
+// parts of 4, 37 of 6, 40 of 8.
+static uint32_t pa_part_chunks(PaGeom geo, uint32_t num_kv) {
+    const uint32_t kCUs = 256, ntiles = (geo.n_tok + geo.TQ - 1) / geo.TQ;
+    uint32_t best = kPaPartChunks, most = kPaPartChunks;
+    double best_cost = 1e30;
+    for (uint32_t P = kPaPartChunks; P <= most; P += 1 + P / 12) {
+        geo.pchunks = P;
+        uint32_t parts = 0, split = 0, longest = 0, chunks = 0;
+        for (uint32_t t = 0; t < ntiles; ++t) {
+            uint32_t cf, ce;
+            pa_chunks(geo, t, cf, ce);
+            const uint32_t np = pa_parts(geo, t), len = (ce - cf + np - 1) / np;
+            parts += np;
+            split += np > 1 ? np : 0;
+            chunks += ce - cf;
+            longest = len > longest ? len : longest;
+            most = ce - cf > most ? ce - cf : most;
+        }
+        const uint32_t wgs = parts * num_kv, rounds = (wgs + kCUs - 1) / kCUs;
+        const double walk = rounds == 1 ? longest : (double)chunks / parts;
+        const double cost = rounds * (walk + 1.2) + 0.0125 * split * num_kv;
+        if (cost < best_cost - 1e-9) {
+            best_cost = cost;
+            best = P;
+        }
+    }
+    return best;
+}
+
 static void launch_pa_merge(hipStream_t st, const float *ws, const PaGeom &geo, uint32_t num_q_heads, uint32_t D,
                             float *out, __bf16 *outb, uint32_t ntt) {
     const size_t nrow = (size_t)geo.n_tok * num_q_heads;
@@ -1323,18 +1364,14 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
             k_prefill_frags<<<dim3(num_kv, c_pre - c_lo, 2), 256, 0, st>>>(kc, vc, slots, n_keys, c_lo, nfch,
                                                                          kv_dim, frag);
         const uint32_t tq = 16 * kPaWaves / gqa;
-        // Causal tiles differ in length (the last one walks every key): each
-        // tile's chunks are cut into parts of about kPaPartChunks chunks (at
-        // most kPaParts), so the longest walk is about that long and the
-        // short tiles run whole (512 tokens: 16 tiles of 1..16 chunks -> 40
-        // parts of at most 4 chunks per KV head).
-        const PaGeom geo{tq, n_tok, num_prev, window, ws ? kPaParts : 1u};
+        PaGeom geo{tq, n_tok, num_prev, window, ws ? kPaParts : 1u, kPaPartChunks};
+        if (ws) geo.pchunks = pa_part_chunks(geo, num_kv);
         uint32_t items = 0;
         const bool split = pa_items(geo, items);
         const dim3 mgrid(num_q_heads / gqa, items);
 #define CHN_PATTN_MF(G)                                                                                  \
     k_prefill_attn_mf<G><<<mgrid, 64 * kPaWaves, 0, st>>>(q, frag, c_lo, nfch, num_prev, n_tok, num_q_heads, scale, \
-                                                         window, out, outb, ws, geo.maxparts, ntt)
+                                                         window, out, outb, ws, geo.maxparts, geo.pchunks, ntt)
         switch (gqa) {
         case 1: CHN_PATTN_MF(1); break;
         case 2: CHN_PATTN_MF(2); break;
@@ -1347,7 +1384,8 @@ int launch_prefill_attn(hipStream_t st, const float *q, const float *kc, const f
     }
     if (head_dim == 512 && (gqa == 1 || gqa == 2 || gqa == 4)) {
         const uint32_t num_kv = num_q_heads / gqa;
-        const PaGeom geo{16 / gqa, n_tok, num_prev, window, ws ? pa5_parts(n_tok, num_prev + n_tok, gqa, num_kv) : 1u};
+        const PaGeom geo{16 / gqa, n_tok, num_prev, window, ws ? pa5_parts(n_tok, num_prev + n_tok, gqa, num_kv) : 1u,
+                         kPaPartChunks};
         uint32_t items = 0;
         const bool split = pa_items(geo, items);
         const dim3 grid(num_kv, items);
