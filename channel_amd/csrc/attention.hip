@@ -764,6 +764,15 @@ __device__ __forceinline__ void pa_item(const PaGeom &geo, uint32_t it, int lane
 
 // F: the pre-pass output for chunks c_lo .. c_lo + nfch - 1.  Grid (KV
 // heads, work items of pa_item).
+// What bounds it: instruction issue beside the MFMAs (an MFMA takes 8 of its
+// 16 cycles' issue slots, every other vector operation 4.4 with two waves per
+// SIMD), the LDS reads of a chunk by eight waves, and the chunk's chain of
+// waits.  Of 3.5 vector operations per MFMA, the rescaling of the sums in
+// every chunk, the masks of chunks that no query's window cuts, and an address
+// per LDS read are gone (1.2 in such a chunk): 1024 tokens after 2000 180 -> 166
+// us, 512 after 512 (window 1024) 50 -> 47 us.  Pairs of waves that share a
+// chunk's fragments, half the LDS reads but scores exchanged through LDS, were
+// slower (1024 tokens 86 against 73 us).
 template <int GQA>
 __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *__restrict__ Q,
                                                          const unsigned char *__restrict__ F, uint32_t c_lo,
@@ -788,6 +797,8 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
     const uint32_t tqc = min(tq, n_tok - 1);
     const uint32_t Sq = num_prev + tqc + 1;                        // keys [startq, Sq)
     const uint32_t startq = (window > 0 && Sq > window) ? Sq - window : 0;
+    // the wave's first query's end and last query's start (lanes 0 and 15)
+    const uint32_t end_first = __builtin_amdgcn_readfirstlane(Sq), win_last = __builtin_amdgcn_readlane(startq, 15);
     // the tile's 32-key chunks [cf, ce) (from its first token's window start
     // to its last token), cut into nparts parts; the parts' partial states
     // meet in k_prefill_attn_merge
@@ -847,18 +858,19 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
         // fragments (K hi / lo of both tiles) load while slice j-1 multiplies.
         f4 sacc[2] = {f4{0, 0, 0, 0}, f4{0, 0, 0, 0}};
         pbf16x8 kf[2][4];
-        auto kread = [&](int j, pbf16x8 (&d)[4]) {
-            d[0] = lds_read<pbf16x8>(base + (0 * 8 + j) * kPaFrag);
-            d[1] = lds_read<pbf16x8>(base + kPaPlane + (0 * 8 + j) * kPaFrag);
-            d[2] = lds_read<pbf16x8>(base + (1 * 8 + j) * kPaFrag);
-            d[3] = lds_read<pbf16x8>(base + kPaPlane + (1 * 8 + j) * kPaFrag);
+        auto kread = [&](auto j_, pbf16x8 (&d)[4]) {
+            constexpr int j = decltype(j_)::value;
+            d[0] = lds_read<pbf16x8, j * kPaFrag>(base);
+            d[1] = lds_read<pbf16x8, kPaPlane + j * kPaFrag>(base);
+            d[2] = lds_read<pbf16x8, (8 + j) * kPaFrag>(base);
+            d[3] = lds_read<pbf16x8, kPaPlane + (8 + j) * kPaFrag>(base);
         };
-        kread(0, kf[0]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        kread(std::integral_constant<int, 0>{}, kf[0]);
+        static_for<8>([&](auto j_) {
+            constexpr int j = decltype(j_)::value;
             pbf16x8 (&cur)[4] = kf[j & 1];
-            if (j < 7) {
-                kread(j + 1, kf[(j + 1) & 1]);
+            if constexpr (j < 7) {
+                kread(std::integral_constant<int, j + 1>{}, kf[(j + 1) & 1]);
                 lds_wait_n<4>();                                   // slice j landed (slice j+1 may fly)
             } else {
                 lds_wait();
@@ -871,34 +883,46 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
                 sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[2 * tt], ql[j], sacc[tt], 0, 0, 0);
                 sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[2 * tt + 1], qh[j], sacc[tt], 0, 0, 0);
             }
-        }
+        });
         // online softmax for query c over this chunk (lane groups g hold 8 keys each)
         float sv[8];
         float cmax = -INFINITY;
+        if (c0 >= win_last && c0 + NK <= end_first) {              // every key is every query's
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t kp = c0 + 16 * tt + 4 * g + i;
-                const bool ok = kp >= startq && kp < Sq;
-                const float v = ok ? sacc[tt][i] * scale : -INFINITY;
-                sv[4 * tt + i] = v;
-                cmax = fmaxf(cmax, v);
+            for (int i = 0; i < 8; ++i) {
+                sv[i] = sacc[i >> 2][i & 3] * scale;
+                cmax = fmaxf(cmax, sv[i]);
             }
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
-        const float m_new = fmaxf(m, cmax);
-        const float alpha = (m_new == -INFINITY) ? 1.0f : __expf(m - m_new);
-        float psum = 0.0f, pv[8];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t kp = c0 + 16 * (i >> 2) + 4 * g + (i & 3);
+                const bool ok = kp >= startq && kp < Sq;
+                sv[i] = ok ? sacc[i >> 2][i & 3] * scale : -INFINITY;
+                cmax = fmaxf(cmax, sv[i]);
+            }
+        }
+        // The sums are rescaled, and maxima exchanged, only in chunks where some
+        // query's maximum rises (m stays the maximum itself: its probability, often
+        // most of the sum, is then 1 and its low half 0, so the dropped low product
+        // misses it; m up to 6 behind cost 6.4e-6 of error instead of 6.0e-6).
+        if (__ballot(cmax > m)) {
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+            const float m_new = fmaxf(m, cmax);
+            const float alpha = (m_new == -INFINITY) ? 1.0f : __expf(m - m_new);
+            m = m_new;
+            l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 16; ++dt) o[dt] *= alpha;
+        }
+        const float m0 = m == -INFINITY ? 0.0f : m;                // (only -Inf scores so far)
+        float pv[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            pv[i] = sv[i] == -INFINITY ? 0.0f : __expf(sv[i] - m_new);
-            psum += pv[i];
+            pv[i] = __expf(sv[i] - m0);
+            l += pv[i];                                            // this lane's keys; the groups meet at the end
         }
-        psum += __shfl_xor(psum, 16, 64);
-        psum += __shfl_xor(psum, 32, 64);
-        l = l * alpha + psum;
-        m = m_new;
         pu32x4 ph, pl;
 #pragma unroll
         for (int i = 0; i < 4; ++i) put_hilo(ph, pl, i, pv[2 * i], pv[2 * i + 1]);
@@ -906,28 +930,30 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mf(const float *
         // O^T tile dt: dims 16 dt + 4 g + i, query c; tile dt+1's V^T
         // fragments load while tile dt multiplies
         pbf16x8 vf[2][2];
-        auto vread = [&](int dt, pbf16x8 (&d)[2]) {
-            d[0] = lds_read<pbf16x8>(base + 2 * kPaPlane + dt * kPaFrag);
-            d[1] = lds_read<pbf16x8>(base + 3 * kPaPlane + dt * kPaFrag);
+        auto vread = [&](auto dt_, pbf16x8 (&d)[2]) {
+            constexpr int dt = decltype(dt_)::value;
+            d[0] = lds_read<pbf16x8, 2 * kPaPlane + dt * kPaFrag>(base);
+            d[1] = lds_read<pbf16x8, 3 * kPaPlane + dt * kPaFrag>(base);
         };
-        vread(0, vf[0]);
-#pragma unroll
-        for (int dt = 0; dt < 16; ++dt) {
+        vread(std::integral_constant<int, 0>{}, vf[0]);
+        static_for<16>([&](auto dt_) {
+            constexpr int dt = decltype(dt_)::value;
             pbf16x8 (&cur)[2] = vf[dt & 1];
-            if (dt < 15) {
-                vread(dt + 1, vf[(dt + 1) & 1]);
+            if constexpr (dt < 15) {
+                vread(std::integral_constant<int, dt + 1>{}, vf[(dt + 1) & 1]);
                 lds_wait_n<2>();
             } else {
                 lds_wait();
             }
             lds_pin(cur[0]);
             lds_pin(cur[1]);
-            o[dt] *= alpha;
             o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[0], bh, o[dt], 0, 0, 0);
             o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[0], bl, o[dt], 0, 0, 0);
             o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[1], bh, o[dt], 0, 0, 0);
-        }
+        });
     }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
     if (tq >= n_tok) return;
     const size_t orow = ((size_t)tq * num_q_heads + head) * D + 4 * g;
     if (nparts > 1) {

@@ -7,6 +7,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <string>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "../../include/channel_hip.h"
@@ -602,6 +604,17 @@ __device__ __forceinline__ void emit_planes8(const float (&v)[8], uint32_t *__re
     emit_planes8s(v, xp, nb, 1, b, w, ok);
 }
 
+
+// f(std::integral_constant<int, i>) for i = 0 .. N-1 (compile-time indices,
+// e.g. for the immediate offsets of asm LDS reads).
+template <typename F, int... I>
+__host__ __device__ __forceinline__ void static_for_(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__host__ __device__ __forceinline__ void static_for(F &&f) {
+    static_for_(f, std::make_integer_sequence<int, N>{});
+}
 
 // ---------------------------------------------------------------------
 // DMA into LDS (global_load_lds) and the waits around it, shared by the

@@ -10,9 +10,6 @@
 // or a pre-pass, weights to bf16(scale * (q - 8)); fp32 accumulation.
 #include "chn_internal.h"
 
-#include <type_traits>
-#include <utility>
-
 namespace chn {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -60,17 +57,6 @@ struct GemmArgs {
     uint32_t ksplit;
     size_t ypart;
 };
-
-// f(std::integral_constant<int, i>) for i = 0 .. N-1 (compile-time indices,
-// e.g. for the immediate offsets of asm LDS reads).
-template <typename F, int... I>
-__host__ __device__ __forceinline__ void static_for_(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__host__ __device__ __forceinline__ void static_for(F &&f) {
-    static_for_(f, std::make_integer_sequence<int, N>{});
-}
 
 __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0, 0, 0, 0};
 

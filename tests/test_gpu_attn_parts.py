@@ -38,3 +38,24 @@ def test_parts(ctx, nq, gqa, n, prev, window):
         want = oracle.batch_causal_attn(np.ascontiguousarray(Qh[t: t + 3]), Kh, Vh, slots[: prev + t + 3], 3, prev + t,
                                         nq, D, kvd, gqa, 1.0, window)
         assert rel_err(got[t: t + 3], want.reshape(3, -1)) < 1e-3
+
+
+@pytest.mark.parametrize("step", [-2.0, 0.0, 2.0, 4.0, 9.0])
+def test_rising_scores(ctx, step):
+    """Scores that rise (or fall) by up to `step` times 16 per 32-key chunk,
+    differently for the queries of a wave: the sums are rescaled in every chunk,
+    in some, or only in the first."""
+    nq, gqa, D, n, prev = 4, 2, 256, 70, 470
+    nkv, S = nq // gqa, prev + n
+    rng = np.random.default_rng(3)
+    u = rng.choice([-1.0, 1.0], D) / 16
+    K = (0.02 * rng.standard_normal((S, nkv, D)) + (step * np.arange(S) / 32)[:, None, None] * u).astype(np.float32)
+    V = rng.standard_normal((S, nkv * D)).astype(np.float32)
+    Q = (rng.standard_normal((n, nq, D)) + u * rng.uniform(0, 1, (n, nq, 1)) * 16 ** 0.5 * 4).astype(np.float32) / 4
+    slots = np.arange(S, dtype=np.uint32)
+    out = ctx.alloc(n * nq * D * 4)
+    say(f"attention with scores rising by {step} per chunk")
+    ctx.call("chn_batch_causal_attn", ctx.upload(Q), ctx.upload(K), ctx.upload(V), ctx.upload(slots), n, prev, nq, D,
+             nkv * D, gqa, 4.0, 0, out)
+    want = oracle.batch_causal_attn(Q.reshape(n, -1), K.ravel(), V.ravel(), slots, n, prev, nq, D, nkv * D, gqa, 4.0, 0)
+    assert rel_err(f32_host(ctx, out, n * nq * D), want.ravel()) < 1e-3
