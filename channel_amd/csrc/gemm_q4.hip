@@ -60,6 +60,23 @@ struct GemmArgs {
 
 __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0, 0, 0, 0};
 
+// Barrier of the four waves that share the LDS counter n: the wave's last LDS
+// reads and its DMA are done (the caller waited), lane 0 counts it in, and it
+// goes on once the count has reached `target`.  The four waves are in one
+// workgroup, so all of them run, and each counts itself in before it waits.
+// With s_barrier the two groups of a G 2 workgroup wait for each other at
+// every slab: q/k/v at 300 tokens 39.1 against 37.2 us, at 512 42.9 against 42.5;
+// o_proj at 300 tokens 31.0 against 30.2, at 700 42.7 against 40.8.
+__device__ __forceinline__ void group_barrier(uint32_t *n, uint32_t target, int lane) {
+    __asm__ volatile("" ::: "memory");
+    if (lane == 0) __hip_atomic_fetch_add(n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while ((int32_t)(__builtin_amdgcn_readfirstlane(
+                         __hip_atomic_load(n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) -
+                     target) < 0) {
+    }
+    __asm__ volatile("" ::: "memory");
+}
+
 // The contraction of one tile: 128 tokens x 64 FT / NMAT features per
 // matrix, four waves (times G) of all 128 tokens x FT feature tiles of 16.
 //
@@ -88,7 +105,7 @@ __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0, 0, 0, 0
 // whose sums meet in LDS, ksplit does so in separate workgroups.
 //
 // Calls at 12B dims with their bf16 pass, before and now, us: 512 x 3840 ->
-// 15360 89 / 72; q/k/v 300 tokens 64 / 39, 512 tokens 51 / 44; gate/up 256
+// 15360 89 / 72; q/k/v 300 tokens 64 / 37, 512 tokens 51 / 43; gate/up 256
 // tokens 120 / 70, 512 tokens 126 / 124; down 512 tokens 97 / 84, 1024 tokens
 // 186 / 150; o_proj 512 tokens 38 / 32, 1024 tokens 69 / 46.
 //
@@ -99,6 +116,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
     constexpr int SLOT = BT * 256, RING = 4, LA = RING - 1;
     constexpr bool kAtOnce = NMAT == 2 && FT == 4 && REP;
     __shared__ __attribute__((aligned(16))) unsigned char sm[2 * G * SLOT];
+    __shared__ uint32_t arrived[2];                            // G 2: waves of a group that passed a slab, counted up
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
     const uint32_t grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
@@ -118,15 +136,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
     ct -= sg == 0 ? 0u : (sg == 1 ? a.c0[1] : a.c0[2]);
     const uint32_t n0 = ct * BN + wave * (16 * NF), t0 = tt * BT;
     const uint32_t K = a.K, nb = K / 32, S = (nb + 3) / 4;
-    // this group's slabs [s0, s1) of the workgroup's share of K; the loop runs
-    // the larger group's count, so that every wave meets every barrier
+    // this group's slabs [s0, s1) of the workgroup's share of K
     const uint32_t ntot = a.ksplit * G, part = ks * G + grp;
     const uint32_t s0 = part * S / ntot, s1 = (part + 1) * S / ntot;
-    uint32_t iters = s1 - s0;
-    if (G == 2) {
-        const uint32_t p2 = ks * 2 + 1 - grp, o = (p2 + 1) * S / ntot - p2 * S / ntot;
-        iters = iters > o ? iters : o;
-    }
     unsigned char *xs = sm + grp * 2 * SLOT;
 
     // X: instruction i of wave w copies rows 16 i + 4 w .. + 3 of the slab, chunk
@@ -201,6 +213,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
     u32x4v A[2][FT];
     bf16x8 xf[RING];
     Raw rc, rn;
+    if (G == 2 && tid < 2) arrived[tid] = 0;
     issue_x(min(s0, S - 1), 0);
 #pragma unroll
     for (int f = 0; f < FT; ++f) load_raw(min(s0, S - 1), rc, f);
@@ -220,18 +233,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
         for (int p = 0; p < 4; ++p) unit(rc.q[f], 0, f, p, A[0][f]);
     }
     uint32_t slot = 0;                                         // byte offset of slab s's X
-    for (uint32_t it = 0; it < iters; ++it) {
-        const uint32_t s = s0 + it;
-        if (G == 2 && s >= s1) {                               // the other group has one slab more
-            bare_barrier();
-            break;
-        }
+    for (uint32_t s = s0; s < s1; ++s) {
         const uint32_t sn = min(s + 1, S - 1);
         static_for<NST>([&](auto i_) {
             constexpr int i = decltype(i_)::value, j = i / NTT, t = i % NTT;
             if constexpr (i == NST - LA) {                     // slab s's last fragments are read
                 wait_vm_lgkm0<0>();                            // ... and slab s + 1's DMA landed
-                bare_barrier();                                // ... for every wave
+                if constexpr (G == 2) group_barrier(&arrived[grp], 4 * (s - s0 + 1), lane);
+                else bare_barrier();                           // ... for every wave of the group
                 if (s + 2 < s1) issue_x(s + 2, slot);
                 slot ^= SLOT;
 #pragma unroll
@@ -339,7 +348,7 @@ __global__ __launch_bounds__(256 * G, 2) void k_q4gemm_p(GemmArgs a) { gemm_tile
 //    tokens 121 against 128 us, but 700 tokens 197 against 188; K % 128 == 0.
 //  * one group from T >= 360 (15360 x 3840, 300 tokens: 65 us, two groups 73);
 //  * below, two groups, whose waves hide each other's waits where a CU has one
-//    workgroup (8192 x 3840, 300 tokens: 39 against 42 us), and below T = 160
+//    workgroup (8192 x 3840, 300 tokens: 37 against 42 us), and below T = 160
 //    K split over two workgroups as well (3840 x 4096, 512 tokens: 26 against
 //    38 us); up to 256 tokens with 64-token tiles, alone if those give 160
 //    workgroups (8192 x 3840, 256 tokens: 34 against 38 us), else in four
