@@ -209,7 +209,7 @@ int chn_ffn_gate_up_q4r(chn_ctx *ctx, const void *Wg, const void *Wu, const floa
 
 /* Y[t][r] = sum_k X[t][k] * W[r][k] for t < n_tok, r < M: X fp32 [n_tok][K]
  * (16-byte aligned), W Q4 [M][K], Y fp32 [n_tok][M].  Operands are rounded
- * to bf16 (X) and bf16(scale*(q-8)) (W, dequantized in LDS) for MFMA with
+ * to bf16 (X) and bf16(scale*(q-8)) (W, dequantized in registers) for MFMA with
  * fp32 accumulation; results match the fp32 contraction within 1e-2
  * relative.  The reference's push constants call n_tok "N" and the output
  * rows "M".  batch_gemm_q4 (shaders/batch_gemm_q4.wgsl; the unreferenced
