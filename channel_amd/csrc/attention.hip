@@ -583,7 +583,7 @@ __device__ __forceinline__ void store_out4(float *out, __bf16 *outb, uint32_t nt
 //
 // An online softmax over each query's causal window (shaders/
 // batch_causal_attn.wgsl: keys [start, prev + t + 1) of the list, start = S -
-// window for window > 0 and S > window), computed per workgroup for 64 query rows (64 / GQA tokens x the
+// window for window > 0 and S > window), computed per workgroup for 128 query rows (128 / GQA tokens x the
 // GQA heads of one KV head) against 32-key chunks of the slot list:
 //  * scores are formed transposed, S^T = K Q^T, with
 //    v_mfma_f32_16x16x32_bf16; each fp32 operand is split into bf16 high

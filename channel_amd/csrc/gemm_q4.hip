@@ -16,6 +16,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 
 // Activations to bf16 (RNE).
@@ -296,7 +297,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
     }
     // epilogue: lane holds features 4g + i of each tile, token r
     float *Yp = Y + ks * a.ypart;
-    const bool vec = M % 4 == 0 && (a.Yb ? ((uintptr_t)a.Yb & 7) == 0 : ((uintptr_t)Yp & 15) == 0);
+    const bool vec = M % 4 == 0 && ((uintptr_t)a.Yb & 7) == 0;
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
@@ -318,9 +319,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
                 }
                 continue;
             }
-            float *y = Yp + (size_t)tok * M + n;
-            if (vec) {
-                *(f32x4 *)y = v;
+            float *y = Yp + (size_t)tok * M + n;                   // (4-byte alignment is enough)
+            if (n + 4 <= M) {
+                *(f32x4_a4 *)y = v;
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
