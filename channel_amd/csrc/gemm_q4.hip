@@ -355,6 +355,11 @@ __global__ __launch_bounds__(256 * G, 2) void k_q4gemm_p(GemmArgs a) { gemm_tile
 //    workgroups (8192 x 3840, 256 tokens: 34 against 38 us), else in four
 //    parts or two times two groups (3840 x 4096, 192 tokens: 24 us, 128-token
 //    tiles 28, one part of 64 x 64 tiles 37).
+//  * Few tiles take the 64-token ones beyond 256 tokens too (T <= 64: 512 x 4096
+//    -> 513 19.3 against 28.1 us, 1024 x 512 -> 1000 10.3 against 12.8), and so
+//    does a K of less than four slabs, whose walk is too short to hide its
+//    prologue (T < 200: 200 x 320 -> 8191 9.5 against 11.5 us, 600 x 320 -> 600
+//    8.2 against 10.1; 500 x 256 -> 5000 10.2 against 9.9).
 //  * Where the caller takes four partial outputs and K is long, splitting over
 //    workgroups alone: down 3840 x 15360 at 512 tokens in four 69, two times
 //    two groups 75 us; with shorter K the partials cost the consumer more.
@@ -365,11 +370,12 @@ struct GemmShape {
 static GemmShape gemm_shape(uint32_t nmat, uint32_t n_tok, uint32_t ct, uint32_t K, uint32_t max_parts) {
     const uint32_t T = ct * ((n_tok + 127) / 128), T4 = T / 2, slabs = (K + 127) / 128;
     if (K % 128 == 0 && T4 >= 448 && (T4 >= 2048 || T4 % 512 >= 448 || T4 % 512 == 0)) return {true, 128, 1, 1};
-    if (nmat == 2 || T >= 360 || slabs < 4) return {false, 128, 1, 1};
+    if (nmat == 2 || T >= 360) return {false, 128, 1, 1};
+    if (slabs < 4) return {false, T < 200 ? 64u : 128u, 1, 1};
     if (max_parts >= 4 && slabs >= 64) return {false, 128, T < 60 ? 2u : 1u, 2 * T >= 360 ? 2u : 4u};
     if (T >= 160) return {false, 128, 2, 1};
     const uint32_t T64 = ct * ((n_tok + 63) / 64);
-    if (n_tok <= 256) {
+    if (n_tok <= 256 || T <= 64) {
         if (T64 >= 160 || slabs < 8 || max_parts < 2) return {false, 64, 1, 1};
         return max_parts >= 4 && slabs >= 16 ? GemmShape{false, 64, 1, 4} : GemmShape{false, 64, 2, 2};
     }
