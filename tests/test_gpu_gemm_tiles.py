@@ -19,9 +19,12 @@ pytestmark = pytest.mark.gpu
     (200, 300, 1056),      # 64-token tiles with K split in two times two, ragged K
     (150, 140, 2080),      # 64-token tiles with K split in four, ragged K
     (65, 200, 8224),       # long K above the wide limit: two groups, K split in four
-    (257, 70, 416),        # 128-token tiles of two groups, one without a last slab
-    (260, 260, 1184),      # two groups and K split in two
-    (300, 7000, 160),      # two groups alone (165 tiles)
+    (257, 70, 416),        # few tiles: 64 tokens beyond 256 too
+    (260, 260, 1184),      # the same with K split
+    (300, 7000, 160),      # fewer than four slabs: 64-token tiles
+    (300, 2903, 544),      # 128-token tiles of two groups, one with a slab less, odd row length
+    (300, 2900, 1056),     # two groups and K split in two
+    (300, 7001, 544),      # two groups alone (165 tiles)
     (385, 11520, 96),      # one group (360 tiles), one ragged slab
     (130, 57300, 128),     # 256-feature tiles (448 of them), one slab
 ])
