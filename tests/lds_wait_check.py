@@ -6,9 +6,12 @@ compiler cannot tell its DMA ring slots apart and would otherwise wait for
 every DMA in flight before each read).  The compiler does not know such an
 asm result is still in flight, so it must not copy, read or overwrite the
 destination registers before the s_waitcnt lgkmcnt that retires the load.
-This scans every function whose name matches a pattern and reports any
-instruction that touches the VGPRs of a pending ds_read (LDS operations
-retire in issue order, so lgkmcnt(n) retires all but the newest n).
+This follows every path through each function whose name matches a pattern
+(reads may be in flight over a loop's back edge, where the compiler may place
+the copies of a rotated loop) and reports any instruction that touches the
+VGPRs of a pending ds_read.  LDS operations retire in issue order, so
+lgkmcnt(n) leaves at most the newest n of them; scalar loads, which share the
+counter and return in any order, are taken as returned already.
 
 usage: python tests/lds_wait_check.py file.s [name-substring]
 """
@@ -20,43 +23,70 @@ def _regs(tok):
     m = re.fullmatch(r"[va]\[(\d+):(\d+)\]", tok)
     if m:
         pre = tok[0]
-        return {(pre, i) for i in range(int(m.group(1)), int(m.group(2)) + 1)}
+        return frozenset((pre, i) for i in range(int(m.group(1)), int(m.group(2)) + 1))
     m = re.fullmatch(r"([va])(\d+)", tok)
     if m:
-        return {(m.group(1), int(m.group(2)))}
-    return set()
+        return frozenset({(m.group(1), int(m.group(2)))})
+    return frozenset()
+
+
+def _parse(lines):
+    """([(line number, text, op, operands)], {label: index of the instruction after it})."""
+    ins, labels = [], {}
+    for ln, raw in lines:
+        t = raw.split(";")[0].strip()
+        m = re.match(r"([.\w$]+):\s*(.*)", t)
+        if m:
+            labels[m.group(1)] = len(ins)
+            t = m.group(2)
+        if not t or t.startswith("."):
+            continue
+        op, _, rest = t.partition(" ")
+        ins.append((ln, t, op, [o.strip().split()[0] for o in rest.split(",") if o.strip()]))
+    return ins, labels
 
 
 def check_function(lines):
     """Returns the list of (line number, text) hazards in one function."""
-    pend = []
-    bad = []
-    for ln, raw in lines:
-        t = raw.split(";")[0].strip()
-        if not t or t.endswith(":") or t.startswith("."):
-            continue
-        op, _, rest = t.partition(" ")
-        ops = [o.strip().split()[0] for o in rest.split(",") if o.strip()] if rest else []
-        if op == "s_waitcnt":
-            m = re.search(r"lgkmcnt\((\d+)\)", rest)
-            if m:
-                n = int(m.group(1))
-                pend = pend[len(pend) - n:] if 0 < n < len(pend) else ([] if n == 0 else pend)
-            continue
-        if op.startswith("s_load") or op.startswith("s_buffer_load"):
-            pend.append(set())
-            continue
-        if op.startswith("s_"):
-            continue
-        live = set().union(*pend) if pend else set()
-        touched = set().union(*[_regs(o) for o in ops]) if ops else set()
-        if touched & live:
-            bad.append((ln, t))
-        if op.startswith("ds_read"):
-            pend.append(_regs(ops[0]) if ops else set())
-        elif op.startswith("ds_"):
-            pend.append(set())
-    return bad
+    ins, labels = _parse(lines)
+    bad = {}
+    work, seen = [(0, ())], set()                       # (instruction, pending loads, oldest first)
+    while work:
+        i, pend = work.pop()
+        while i < len(ins):
+            ln, t, op, ops = ins[i]
+            i += 1
+            if op == "s_endpgm":
+                break
+            if op in ("s_setpc_b64", "s_swappc_b64", "s_call_b64"):
+                bad[ln] = t + " (a jump that is not followed)"
+                break
+            if op == "s_branch" or op.startswith("s_cbranch"):
+                target = labels.get(ops[-1])
+                if target is None:
+                    bad[ln] = t + " (unknown label)"
+                    break
+                # both ways are joints, so that every loop meets a state it has seen
+                for nxt in (target,) if op == "s_branch" else (target, i):
+                    if (nxt, pend) not in seen:
+                        seen.add((nxt, pend))
+                        work.append((nxt, pend))
+                break
+            if op == "s_waitcnt":
+                m = re.search(r"lgkmcnt\((\d+)\)", t)
+                if m:
+                    n = int(m.group(1))
+                    pend = pend[max(0, len(pend) - n):] if n else ()
+                continue
+            if op.startswith("s_"):
+                continue
+            touched = frozenset().union(*map(_regs, ops))
+            if any(touched & p for p in pend):
+                bad[ln] = t
+            if op.startswith("ds_"):
+                pend += (_regs(ops[0]) if op.startswith("ds_read") and ops else frozenset(),)
+                pend = pend[-64:]                       # (the counter stalls the wave long before that)
+    return sorted(bad.items())
 
 
 def check_file(path, pattern=""):
@@ -68,10 +98,10 @@ def check_file(path, pattern=""):
             cur = m.group(1)
             funcs[cur] = []
             continue
+        if line.startswith(".Lfunc_end"):
+            cur = None
         if cur is not None:
             funcs[cur].append((i, line))
-            if "s_endpgm" in line:
-                cur = None
     return {f: check_function(ls) for f, ls in funcs.items() if pattern in f}
 
 

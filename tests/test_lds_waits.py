@@ -28,10 +28,56 @@ def test_gemm_lds_waits(tmp_path):
     assert len(res2) == 2, "expected both layouts of the DMA-fed gate/up"
     res.update(res2)
     res3 = lds_wait_check.check_file(str(out), "k_q4gemm2s")
-    assert len(res3) == 2, "expected both layouts of the 256-token single-matrix contraction"
+    assert len(res3) == 2, "expected both layouts of the 256-feature single-matrix contraction"
     res.update(res3)
     bad = {f: h for f, h in res.items() if h}
     assert not bad, bad
+
+
+LOOP = """
+_Zk:
+        ds_read_b128 v[0:3], v8
+        s_waitcnt lgkmcnt(0)
+        {enter}
+.LBB0_1:
+        {head}
+        ds_read_b128 v[4:7], v8 offset:16
+        s_waitcnt lgkmcnt(1)
+        v_add_f32_e32 v9, v0, v1
+        {tail}
+        ds_read_b128 v[0:3], v8 offset:32
+        s_waitcnt lgkmcnt(1)
+        v_add_f32_e32 v9, v4, v5
+        s_cbranch_scc1 .LBB0_1
+        s_branch .LBB0_3
+.LBB0_2:
+        {behind}
+        s_branch .LBB0_1
+.LBB0_3:
+        {exit}
+        s_endpgm
+.Lfunc_end0:
+"""
+
+
+@pytest.mark.parametrize("at,what,bad", [
+    ("enter", "s_branch .LBB0_2", 0),                    # a loop entered through a block behind it
+    ("head", "v_mov_b32_e32 v10, v2", 1),                # a copy at the loop's head, read in flight over the back edge
+    ("tail", "v_mov_b32_e32 v0, v9", 0),                 # its registers are free between the wait and the next read
+    ("tail", "s_load_dwordx2 s[0:1], s[2:3], 0x0", 0),
+    ("behind", "v_mov_b32_e32 v10, v2", 0),              # never reached with a read in flight
+    ("exit", "v_add_f32_e32 v9, v3, v3", 1),             # past the loop
+    ("exit", "s_waitcnt lgkmcnt(0)\n        v_add_f32_e32 v9, v3, v3", 0),
+    ("exit", "s_waitcnt vmcnt(0)\n        v_mov_b32_e32 v3, 0", 1),
+    ("head", "s_load_dword s0, s[2:3], 0x0\n        s_waitcnt lgkmcnt(1)\n        v_mov_b32_e32 v10, v2", 1),
+])
+def test_checker_follows_branches(tmp_path, at, what, bad):
+    """Mistakes planted in a hand-written loop that keeps a read in flight over
+    its back edge (scalar loads may return first, so they retire no read)."""
+    import lds_wait_check
+    f = tmp_path / "loop.s"
+    f.write_text(LOOP.format(**{k: what if k == at else "" for k in ("enter", "head", "tail", "behind", "exit")}))
+    assert len(lds_wait_check.check_file(str(f))["_Zk"]) == bad
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
