@@ -143,19 +143,29 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
     unsigned char *xs = sm + grp * 2 * SLOT;
 
     // X: instruction i of wave w copies rows 16 i + 4 w .. + 3 of the slab, chunk
-    // c of row t to position c ^ (t & 15) (rows past the last token clamped:
-    // their columns are not stored)
+    // c of row t to position c ^ (t & 15).  Rows past the last token (their
+    // columns are not stored) are clamped: the tile's last group of 16 rows with a
+    // token in it, group gl, has lane offsets of its own, and the groups after it
+    // copy it again.  A group's offset is scalar (64 bits: K may be any width), so
+    // the addresses take two registers.  With an offset per group three of the four
+    // FT 4 kernels spilled 10 to 16 registers in the K loop, each reload a wait for
+    // the DMA issued before it: one matrix 15360 x 3840 at 1024 tokens 133 (Q4R) and
+    // 159 us (Q4) against 123 and 129, gate/up on Q4 at 512 tokens 148 against 129.
     const uint32_t xrow = 4 * wave + (lane >> 4), chunk = (lane & 15) ^ (xrow & 15);
     const __bf16 *Xt = a.X + (size_t)t0 * K;
-    const uint32_t rlim = a.n_tok - 1 - t0;
-    auto xe = [&](int i) { return (min(16 * i + xrow, rlim) * K + chunk * 8) * 2; };
+    const uint32_t rlim = a.n_tok - 1 - t0, gl = rlim / 16;
+    const uint32_t xo = (xrow * K + chunk * 8) * 2, xol = (min(xrow, rlim - 16 * gl) * K + chunk * 8) * 2;
     auto issue_x = [&](uint32_t s, uint32_t slot) {            // slot: byte offset
         const unsigned char *Xs = (const unsigned char *)(Xt + (size_t)s * 128);
         const bool zero = RAG && s * 128 + chunk * 8 >= K;     // past the row's end (K % 128 != 0)
+        uint32_t g1 = gl;
+        if (FT == 4) __asm__ volatile("" : "+s"(g1));          // select per slab: hoisted, the offsets would stay live
 #pragma unroll
-        for (int i = 0; i < NTT; ++i)
-            __builtin_amdgcn_global_load_lds(zero ? (const unsigned char *)g_zero16 : Xs + xe(i),
+        for (int i = 0; i < NTT; ++i) {
+            const unsigned char *Xg = Xs + (size_t)min((uint32_t)i, g1) * 32 * K;
+            __builtin_amdgcn_global_load_lds(zero ? (const unsigned char *)g_zero16 : Xg + ((uint32_t)i < g1 ? xo : xol),
                                              (lds_t *)(xs + slot + (wave + 4 * i) * 1024), 16, 0, 0);
+        }
     };
     struct Raw {
         u32x4v q[FT];
@@ -171,10 +181,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
         Wb[m] = W + (size_t)nr * nb * (REP ? 16 : 20);
         Sb[m] = W + (size_t)M * nb * 16 + (size_t)nr * nb * 2;
     }
-    const uint32_t nr0 = min(n0, M - 1);
+    const uint32_t nlim = M - 1 - min(n0, M - 1);
+    const uint32_t wgl = __builtin_amdgcn_readfirstlane(nlim / 16), wr = r * nb, wrl = min(r, nlim - 16 * wgl) * nb;
     auto load_raw = [&](uint32_t s, Raw &w, int f) {
         const uint32_t b = RAG ? min(4 * s + g, nb - 1) : 4 * s + g;
-        const uint32_t o = (min(n0 + f % NF * 16 + r, M - 1) - nr0) * nb + b;
+        uint32_t o;
+        if (NF == 4) {                                         // as X's rows: two lane offsets for the four tiles
+            uint32_t g1 = wgl;
+            __asm__ volatile("" : "+s"(g1));
+            o = min((uint32_t)(f % NF), g1) * 16 * nb + ((uint32_t)(f % NF) < g1 ? wr : wrl) + b;
+        } else {
+            o = min(f % NF * 16 + r, nlim) * nb + b;
+        }
         if (REP) {
             w.q[f] = *(const u32x4v *)(Wb[f / NF] + o * 16);
             w.s[f] = *(const uint16_t *)(Sb[f / NF] + o * 2);

@@ -27,6 +27,8 @@ pytestmark = pytest.mark.gpu
     (300, 7001, 544),      # two groups alone (165 tiles)
     (385, 11520, 96),      # one group (360 tiles), one ragged slab
     (130, 57300, 128),     # 256-feature tiles (448 of them), one slab
+    (130, 57300, 384),     # an odd and an even number of slabs: both DMA slots, the hand-over of the weights
+    (250, 57100, 512),     # (the last group of tokens and of features partly and wholly past the end)
 ])
 def test_gemm_launch_shapes(ctx, n_tok, M, K, repacked):
     W = synth_q4_dev(ctx, M, K, 60 + M)
@@ -48,7 +50,7 @@ def test_gemm_launch_shapes(ctx, n_tok, M, K, repacked):
 
 
 @pytest.mark.parametrize("repacked", [False, True])
-@pytest.mark.parametrize("n_tok,M,K", [(65, 200, 352), (130, 28610, 128)])
+@pytest.mark.parametrize("n_tok,M,K", [(65, 200, 352), (130, 28610, 128), (130, 28610, 384), (245, 28600, 256)])
 def test_gate_up_launch_shapes(ctx, n_tok, M, K, repacked):
     """64 and (448 tiles, K % 128 == 0) 128 features of each matrix per workgroup."""
     W, Wh = [], []
@@ -71,6 +73,24 @@ def test_gate_up_launch_shapes(ctx, n_tok, M, K, repacked):
     g, u = (oracle.batch_gemm_q4_bf16(w, Xh, n_tok, M, K, oracle.NTHREADS) for w in Wh)
     want = oracle.gelu_tanh(g.ravel()).reshape(n_tok, M) * u
     assert rel_err(f32_host(ctx, Y, n_tok * M).reshape(n_tok, M), want) < 1e-4
+
+
+def test_qkv_wide_tiles(ctx):
+    """Three segments on 256-feature tiles (512 of them), several slabs."""
+    n_tok, K, rows = 1020, 384, (8190, 4095, 4095)
+    X = synth_normal_dev(ctx, n_tok * K, 69)
+    Xh = f32_host(ctx, X, n_tok * K).reshape(n_tok, K)
+    R, Wh, Y = [], [], [ctx.alloc(n_tok * M * 4) for M in rows]
+    for i, M in enumerate(rows):
+        w = synth_q4_dev(ctx, M, K, 70 + i)
+        Wh.append(q4_host(ctx, w, M, K))
+        R.append(ctx.alloc(ca.q4r_bytes(M, K)))
+        ctx.call("chn_q4_repack", w, M, K, R[-1])
+    say(f"qkv n_tok={n_tok} rows={rows} K={K}")
+    ctx.call("chn_batch_qkv_q4r", *R, X, *Y, n_tok, rows[0], rows[1], K)
+    for w, y, M in zip(Wh, Y, rows):
+        want = oracle.batch_gemm_q4_bf16(w, Xh, n_tok, M, K, oracle.NTHREADS)
+        assert rel_err(f32_host(ctx, y, n_tok * M).reshape(n_tok, M), want) < 1e-4
 
 
 def test_nonfinite_activations_stay_in_their_row(ctx):

@@ -91,6 +91,17 @@ def test_prefill_attn_lds_waits(tmp_path):
     assert not bad, bad
 
 
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_gemm_kernels_use_no_scratch(tmp_path):
+    """A spilled address of the contractions' K loop is reloaded between DMAs and
+    waits for them; the kernels fit their registers."""
+    import re
+    asm = _compile("gemm_q4.hip", tmp_path / "gemm_q4.s")
+    kernels = re.findall(r"\.name:\s+(\S*k_q4gemm\S*)\n(?:.*\n)*?\s*\.private_segment_fixed_size:\s+(\d+)", asm)
+    assert len(kernels) >= 20
+    assert not [k for k in kernels if k[1] != "0"]
+
+
 def _compile(src, out):
     cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
            "-packed-fp32-ops", "-fno-gpu-rdc", "--cuda-device-only", "-S", os.path.join(CSRC, src), "-o", str(out)]
