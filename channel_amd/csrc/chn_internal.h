@@ -26,6 +26,9 @@ struct chn_ctx {
     void *ws = nullptr;
     size_t ws_bytes = 0;
     uint64_t ws_gen = 0;
+    // The contractions' own scratch (kGemmScratch bytes, for the context's
+    // life): split-K partial sums and few-token activations.
+    void *gemm_scratch = nullptr;
     bool recording = false;     // between chn_record_begin and chn_record_end
     std::vector<chn_recording *> recs;   // live recordings, released by chn_destroy
 };
@@ -266,10 +269,17 @@ int launch_quantize(hipStream_t st, int q8, const uint16_t *src, uint32_t *dst, 
 // limits are where the two meet at 12B dims (both with their bf16 pass, us):
 // gate/up 48 tokens 38 / 44, 64 tokens 43 / 44, 80 tokens 51 / 46; long K
 // (down) 48 tokens 31 / 40, 65 tokens 50 / 40; q/k/v 128 tokens 27 / 36.
-constexpr uint32_t kFewTokens = 128, kFewTokensWide = 64;
+// kFewMaxK: kFewTokensWide rows of it fit the contractions' scratch.
+constexpr uint32_t kFewTokens = 128, kFewTokensWide = 64, kFewMaxK = 1u << 18;
 inline bool few_tokens(uint32_t n_tok, int nmat, uint32_t K) {
-    return n_tok <= (nmat == 2 || K >= 8192 ? kFewTokensWide : kFewTokens);
+    return n_tok <= (nmat == 2 || K >= 8192 ? kFewTokensWide : kFewTokens) && K <= kFewMaxK;
 }
+// What a public contraction needs beyond the n_tok x K bf16 activations of
+// the context workspace lies in ctx->gemm_scratch, which every context has
+// from its creation: the workspace's need grows with n_tok x K alone, so a
+// program that ran its largest batch can record any smaller one, whichever
+// kernel and split that one takes.
+constexpr size_t kGemmScratch = (size_t)48 << 20;
 inline uint32_t xb_tiles(uint32_t n_tok) { return (n_tok + 15) / 16; }
 // xb_at's ntt for the activations of a contraction of n_tok tokens.
 inline uint32_t xb_layout(uint32_t n_tok, int nmat, uint32_t K) {

@@ -446,9 +446,9 @@ static uint32_t gemm_cols(int nmat, int nseg, const uint32_t *M) {
 }
 
 // nseg matrices over the same activations (nmat 1), or gate and up.  A shape
-// that splits K writes the parts to po's buffers (Y[0] and on) if there are
-// enough, else to scratch, from where they are summed
-// into Y[0]; with neither it is not split.
+// that splits K writes the parts to scratch (kGemmScratch bytes), from where
+// they are summed into Y[0], or to po's buffers (Y[0] and on); with neither it
+// is not split.
 static int gemm_run(chn_ctx *ctx, int nmat, int nseg, const float *X, const uint32_t *const *W, const uint32_t *W1,
                     float *const *Y, const uint32_t *M, uint32_t n_tok, uint32_t K, __bf16 *xb, bool repacked,
                     __bf16 *Yb, PartialOut *po, float *scratch) {
@@ -475,7 +475,9 @@ static int gemm_run(chn_ctx *ctx, int nmat, int nseg, const float *X, const uint
     a.n_tok = n_tok;
     a.K = K;
     const uint32_t max_parts = nseg > 1 ? 1 : (scratch ? 4 : (po ? po->max_parts : 1));
-    const GemmShape sh = gemm_shape(nmat, n_tok, gemm_cols(nmat, nseg, M), K, max_parts);
+    GemmShape sh = gemm_shape(nmat, n_tok, gemm_cols(nmat, nseg, M), K, max_parts);
+    // (fits by the rule: it splits less than 360 tiles of 64 KB in two, less than 180 in four)
+    if (scratch && (size_t)sh.ksplit * n_tok * M[0] * 4 > kGemmScratch) sh.ksplit = 1;
     if (sh.ksplit > 1 && scratch) {
         a.Y[0] = scratch;
         a.ypart = (size_t)n_tok * M[0];
@@ -519,6 +521,17 @@ int launch_q4gemm_qkv(chn_ctx *ctx, const float *X, const uint32_t *Wq, const ui
     return gemm_run(ctx, 1, 3, X, W, nullptr, Y, M, n_tok, K, xb, true, nullptr, nullptr, nullptr);
 }
 
+// The public calls' buffer for the bf16 activations (kGemmScratch).
+static int public_activations(chn_ctx *ctx, uint32_t n_tok, int nmat, uint32_t K, __bf16 *&xb) {
+    if (few_tokens(n_tok, nmat, K)) {
+        xb = (__bf16 *)ctx->gemm_scratch;
+        return CHN_OK;
+    }
+    const int rc = ensure_workspace(ctx, (size_t)n_tok * K * 2);
+    xb = (__bf16 *)ctx->ws;
+    return rc;
+}
+
 static int gemm_common(chn_ctx *ctx, int nmat, const uint32_t *W0, const uint32_t *W1, const float *X, float *Y,
                        uint32_t n_tok, uint32_t M, uint32_t K, bool repacked = false, __bf16 *Yb = nullptr) {
     CHN_REQUIRE(ctx, W0 && X && (Y || Yb) && (nmat == 1 || W1), "NULL argument");
@@ -527,13 +540,10 @@ static int gemm_common(chn_ctx *ctx, int nmat, const uint32_t *W0, const uint32_
     CHN_REQUIRE(ctx, aligned(W0, repacked ? 16 : 4) && (!W1 || aligned(W1, repacked ? 16 : 4)),
                 "weights must be %d-byte aligned", repacked ? 16 : 4);
     if (!n_tok || !M) return CHN_OK;
-    // workspace: the bf16 activations, then the partial outputs of a split K
-    const size_t xbytes = (xb_elems(n_tok, K, nmat) * 2 + 255) / 256 * 256;
-    const uint32_t parts = few_tokens(n_tok, nmat, K) ? 1 : gemm_shape(nmat, n_tok, gemm_cols(nmat, 1, &M), K, 4).ksplit;
-    int rc = ensure_workspace(ctx, xbytes + (parts > 1 ? (size_t)parts * n_tok * M * 4 : 0));
+    __bf16 *xb = nullptr;
+    int rc = public_activations(ctx, n_tok, nmat, K, xb);
     if (rc) return rc;
-    float *scratch = parts > 1 ? (float *)((unsigned char *)ctx->ws + xbytes) : nullptr;
-    return gemm_run(ctx, nmat, 1, X, &W0, W1, &Y, &M, n_tok, K, (__bf16 *)ctx->ws, repacked, Yb, nullptr, scratch);
+    return gemm_run(ctx, nmat, 1, X, &W0, W1, &Y, &M, n_tok, K, xb, repacked, Yb, nullptr, (float *)ctx->gemm_scratch);
 }
 
 }  // namespace chn
@@ -576,8 +586,9 @@ extern "C" int chn_batch_qkv_q4r(chn_ctx *ctx, const void *Wq, const void *Wk, c
     CHN_REQUIRE(ctx, K > 0 && K % 32 == 0, "K=%u must be a positive multiple of 32", K);
     CHN_REQUIRE(ctx, aligned(X, 16) && aligned(Wq, 16) && aligned(Wk, 16) && aligned(Wv, 16), "misaligned argument");
     if (!n_tok || !q_dim || !kv_dim) return CHN_OK;
-    int rc = ensure_workspace(ctx, xb_elems(n_tok, K, 1) * 2);
+    __bf16 *xb = nullptr;
+    int rc = public_activations(ctx, n_tok, 1, K, xb);
     if (rc) return rc;
     return launch_q4gemm_qkv(ctx, X, (const uint32_t *)Wq, (const uint32_t *)Wk, (const uint32_t *)Wv, Yq, Yk, Yv,
-                             n_tok, q_dim, kv_dim, K, (__bf16 *)ctx->ws);
+                             n_tok, q_dim, kv_dim, K, xb);
 }

@@ -92,8 +92,10 @@ extern "C" int chn_init(int device, chn_ctx **out) {
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&ctx->t0);
     if (e == hipSuccess) e = hipEventCreate(&ctx->t1);
+    if (e == hipSuccess) e = hipMalloc(&ctx->gemm_scratch, kGemmScratch);
     if (e != hipSuccess) {
-        int rc = hip_fail(nullptr, e, "stream/event create");
+        int rc = hip_fail(nullptr, e, "stream/event/scratch create");
+        if (ctx->t1) (void)hipEventDestroy(ctx->t1);
         if (ctx->t0) (void)hipEventDestroy(ctx->t0);
         if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
         delete ctx;
@@ -134,6 +136,7 @@ extern "C" void chn_destroy(chn_ctx *ctx) {
     ctx->recs.clear();
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->ws) (void)hipFree(ctx->ws);
+    if (ctx->gemm_scratch) (void)hipFree(ctx->gemm_scratch);
     (void)hipEventDestroy(ctx->t0);
     (void)hipEventDestroy(ctx->t1);
     (void)hipStreamDestroy(ctx->stream);

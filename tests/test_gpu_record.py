@@ -104,3 +104,32 @@ def test_recording_misuse_is_refused():
         live = c2.record_end()
         live.submit()
         c2._recs.remove(live)
+
+
+@pytest.mark.parametrize("M,K,largest,smaller", [
+    (3840, 4096, 1024, [640, 256, 129]),     # no split of K at 1024 tokens, in two or four parts below
+    (4, 8224, 65, [64, 17]),                 # few-token activations are padded to 256 columns
+    (4, 4128, 131, [128, 100]),
+])
+def test_smaller_batches_need_no_larger_workspace(M, K, largest, smaller):
+    """A program that ran its largest batch records smaller ones of the same
+    matrix, and eager smaller ones leave its recordings valid."""
+    with Context(0) as c2:
+        W = synth_q4_dev(c2, M, K, 940)
+        X = synth_normal_dev(c2, largest * K, 941)
+        Y = c2.alloc(largest * M * 4)
+        say(f"record: {M} x {K}, {largest} tokens, then {smaller}")
+        c2.call("chn_batch_gemm_q4", W, X, Y, largest, M, K)
+        recs, want = [], []
+        for n in smaller:
+            c2.record_begin()
+            c2.call("chn_batch_gemm_q4", W, X, Y, n, M, K)
+            recs.append(c2.record_end())
+        for n in smaller:
+            c2.call("chn_batch_gemm_q4", W, X, Y, n, M, K)
+            want.append(f32_host(c2, Y, n * M))
+        for _ in range(2):
+            for n, rec, w in zip(smaller, recs, want):
+                c2.fill_u32(Y, 0x7FC00000, n * M)
+                rec.submit()
+                assert np.array_equal(f32_host(c2, Y, n * M), w), n
