@@ -265,14 +265,36 @@ int launch_embed(hipStream_t st, const uint16_t *table, const uint32_t *tokens, 
                  float *x);
 int launch_quantize(hipStream_t st, int q8, const uint16_t *src, uint32_t *dst, uint64_t nblk);
 // Contractions of few tokens run on gemm_q4_few.hip, whose bf16 activations
-// lie in operand order (xb_at); larger ones read them row by row.  The
-// limits are where the two meet at 12B dims (both with their bf16 pass, us):
-// gate/up 48 tokens 38 / 44, 64 tokens 43 / 44, 80 tokens 51 / 46; long K
-// (down) 48 tokens 31 / 40, 65 tokens 50 / 40; q/k/v 128 tokens 27 / 36.
-// kFewMaxK: kFewTokensWide rows of it fit the contractions' scratch.
-constexpr uint32_t kFewTokens = 128, kFewTokensWide = 64, kFewMaxK = 1u << 18;
-inline bool few_tokens(uint32_t n_tok, int nmat, uint32_t K) {
-    return n_tok <= (nmat == 2 || K >= 8192 ? kFewTokensWide : kFewTokens) && K <= kFewMaxK;
+// lie in operand order (xb_at); larger ones read them row by row.  `rows`: all
+// features of the launch, of nseg matrices (a launch of several cannot split K
+// in gemm_q4.hip).  The limits are where the two meet (both with their bf16
+// pass, us, few / larger):
+//  * two matrices or long K: gate/up at 12B dims 48 tokens 38 / 44, 64 tokens
+//    43 / 44, 80 tokens 51 / 46; down 48 tokens 31 / 40, 65 tokens 50 / 40;
+//  * else what counts is the rounds of workgroups (a CU holds one or two of
+//    them): up to 128 tokens 3840 x 4096 (480 of them) 80 tokens 17.7 / 19.9,
+//    100 tokens 21.6 / 18.6, 2048 x 4096 (256) 100 tokens 17.0 / 20.7, 5120 x
+//    2048 (640) 100 tokens 20.3 / 16.9, q/k/v of 8192 rows (512) 128 tokens
+//    21.0 / 26.8, of 10240 (640) 100 tokens 17.6 / 12.2;
+//  * beyond, where K is so short that the larger kernels' third launch or
+//    empty CUs show: 1024 x 1024 129 tokens 6.8 / 11.3, 512 tokens 12.7 /
+//    13.5, 2048 x 1024 256 tokens 11.7 / 13.2; 1024 x 256 350 tokens 8.4 / 7.7,
+//    1536 x 2048 256 tokens 15.9 / 15.8.
+// kFewMaxK: 64 rows of it fit the contractions' scratch.
+constexpr uint32_t kFewMaxTokens = 512, kFewMaxK = 1u << 18;
+inline uint32_t xb_tiles(uint32_t n_tok) { return (n_tok + 15) / 16; }
+// Features per workgroup and matrix: 32 where that leaves about one workgroup
+// per CU.
+inline uint32_t few_features(uint32_t rows) { return rows / 32 >= 240 ? 32 : 16; }
+inline bool few_tokens(uint32_t n_tok, int nmat, uint32_t K, uint32_t rows, int nseg = 1) {
+    if (K > kFewMaxK) return false;
+    if (n_tok <= 64) return true;
+    if (nmat == 2 || K >= 8192 || n_tok > kFewMaxTokens) return false;
+    const uint32_t per = few_features(rows);
+    const uint64_t wgs = (uint64_t)((rows + per - 1) / per) * ((xb_tiles(n_tok) + 3) / 4);
+    if (n_tok > 128) return K >= 512 && K <= 1024 && wgs <= 512;
+    if (nseg > 1) return wgs <= 512;
+    return wgs <= (K <= 2048 ? (n_tok <= 80 ? 640 : 512) : (n_tok <= 80 ? 512 : 256));
 }
 // What a public contraction needs beyond the n_tok x K bf16 activations of
 // the context workspace lies in ctx->gemm_scratch, which every context has
@@ -280,15 +302,12 @@ inline bool few_tokens(uint32_t n_tok, int nmat, uint32_t K) {
 // program that ran its largest batch can record any smaller one, whichever
 // kernel and split that one takes.
 constexpr size_t kGemmScratch = (size_t)48 << 20;
-inline uint32_t xb_tiles(uint32_t n_tok) { return (n_tok + 15) / 16; }
 // xb_at's ntt for the activations of a contraction of n_tok tokens.
-inline uint32_t xb_layout(uint32_t n_tok, int nmat, uint32_t K) {
-    return few_tokens(n_tok, nmat, K) ? xb_tiles(n_tok) : 0u;
+inline uint32_t xb_layout(uint32_t n_tok, int nmat, uint32_t K, uint32_t rows, int nseg = 1) {
+    return few_tokens(n_tok, nmat, K, rows, nseg) ? xb_tiles(n_tok) : 0u;
 }
-// Elements of the bf16 activation buffer of n_tok tokens of width K.
-inline size_t xb_elems(uint32_t n_tok, uint32_t K, int nmat) {
-    return few_tokens(n_tok, nmat, K) ? (size_t)xb_tiles(n_tok) * 16 * ((K + 255) / 256) * 256 : (size_t)n_tok * K;
-}
+// Elements of a bf16 activation buffer that takes either order.
+inline size_t xb_elems(uint32_t n_tok, uint32_t K) { return (size_t)xb_tiles(n_tok) * 16 * ((K + 255) / 256 * 256); }
 // Element (token t, k) of bf16 activations of `width` columns: row-major
 // when ntt is 0, else operand order of k_q4gemm_few over ntt tiles of 16
 // tokens: per 256 K, per half h (the 32-blocks 2g + h), per tile, per word j
@@ -308,9 +327,9 @@ int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const 
                       __bf16 *Yb = nullptr, uint32_t yb_ntt = 0);
 // W0/W1 in the reference Q4 layout, or in Q4R with repacked.  X (fp32) is
 // converted into xb (xb_elems); with X == NULL, xb already holds the bf16
-// activations, in xb_at order for xb_layout(n_tok, nmat, K).
+// activations, in xb_at order for xb_layout.
 // Yb (two-matrix form only): the result goes to Yb as bf16 instead of Y,
-// in the order of a one-matrix contraction when X == NULL, else row-major.
+// in xb_at order for yb_ntt.
 // po (single matrix): a shape that splits K may store its partial sums to
 // Y + p * po->stride, p < po->max_parts (1, 2 or 4), instead of summing them
 // itself; po->parts tells how many it wrote (their sum, in index order, is
@@ -322,7 +341,7 @@ struct PartialOut {
 };
 int launch_q4gemm(chn_ctx *ctx, int nmat, const float *X, const uint32_t *W0, const uint32_t *W1, float *Y,
                   uint32_t n_tok, uint32_t M, uint32_t K, __bf16 *xb, bool repacked, __bf16 *Yb = nullptr,
-                  PartialOut *po = nullptr);
+                  PartialOut *po = nullptr, uint32_t yb_ntt = 0);
 // q, k, v (Q4R) over the same activations in one launch (X == NULL: xb
 // already holds them).
 int launch_q4gemm_qkv(chn_ctx *ctx, const float *X, const uint32_t *Wq, const uint32_t *Wk, const uint32_t *Wv,

@@ -359,45 +359,66 @@ __global__ __launch_bounds__(256, 2) void k_q4gemm2s(GemmArgs a) { gemm_tile<1, 
 template <int NMAT, int BT, int G, bool REP, bool RAG>
 __global__ __launch_bounds__(256 * G, 2) void k_q4gemm_p(GemmArgs a) { gemm_tile<NMAT, BT, 2, G, REP, RAG>(a); }
 
-// Launch shape of one contraction, from sweeps at 12B dims over 129..1024
-// tokens.  T is the number of 128-token x 128-feature tiles (64 + 64 for two
-// matrices); two workgroups of one group fit a CU.
+// Launch shape of one contraction.  T is the number of 128-token x 128-feature
+// tiles (64 + 64 for two matrices); two workgroups of one group fit a CU.
 //  * FT 4 tiles (half the X reads per MFMA, 3-6 % faster when the chip is
 //    full) where T / 2 of them fill the last round of 512 to 7/8: gate/up 512
 //    tokens 121 against 128 us, but 700 tokens 197 against 188; K % 128 == 0.
-//  * one group from T >= 360 (15360 x 3840, 300 tokens: 65 us, two groups 73);
-//  * below, two groups, whose waves hide each other's waits where a CU has one
-//    workgroup (8192 x 3840, 300 tokens: 37 against 42 us), and below T = 160
-//    K split over two workgroups as well (3840 x 4096, 512 tokens: 26 against
-//    38 us); up to 256 tokens with 64-token tiles, alone if those give 160
-//    workgroups (8192 x 3840, 256 tokens: 34 against 38 us), else in four
-//    parts or two times two groups (3840 x 4096, 192 tokens: 24 us, 128-token
-//    tiles 28, one part of 64 x 64 tiles 37).
-//  * Few tiles take the 64-token ones beyond 256 tokens too (T <= 64: 512 x 4096
-//    -> 513 19.3 against 28.1 us, 1024 x 512 -> 1000 10.3 against 12.8), and so
-//    does a K of less than four slabs, whose walk is too short to hide its
-//    prologue (T < 200: 200 x 320 -> 8191 9.5 against 11.5 us, 600 x 320 -> 600
-//    8.2 against 10.1; 500 x 256 -> 5000 10.2 against 9.9).
-//  * Where the caller takes four partial outputs and K is long, splitting over
-//    workgroups alone: down 3840 x 15360 at 512 tokens in four 69, two times
-//    two groups 75 us; with shorter K the partials cost the consumer more.
+//  * 128-token tiles of one group from T >= 360 (15360 x 3840, 300 tokens: 65
+//    us, two groups 73) and for two matrices.
+//  * Below, tiles of 64 or 128 tokens, one or two groups of waves and K in up
+//    to four parts by shape_us's estimate.
 struct GemmShape {
     bool ft4;
     uint32_t bt, groups, ksplit;
 };
-static GemmShape gemm_shape(uint32_t nmat, uint32_t n_tok, uint32_t ct, uint32_t K, uint32_t max_parts) {
+// The time in us in which the shapes of one matrix differ: rounds of workgroups
+// over the CUs, each the start of a tile and its walk over the slabs, a slab in
+// the time of a lone wave per SIMD or, where more, that of the waves which share
+// it (a CU holds 4 waves per SIMD of 64-token tiles, 2 of 128-token ones); the
+// two groups' meeting; the partial outputs, written and read again, and the launch
+// that sums them if the caller does not (summed).  The constants are fitted to
+// 18000 calls of 1932 sizes (256..24576 rows, K 128..15360, 65..1024 tokens, both
+// layouts): 5 % rms, and the shape it picks is 1 % slower than the best one on
+// average.  us, by thresholds on T as before and now: 2048 x 1024 1024 tokens
+// 25.7 / 15.6, 3840 x 1024 512 tokens 23.1 / 14.3, 3840 x 4096 256 tokens 27.7 /
+// 25.9, 8192 x 4096 256 tokens 39.2 / 33.2, q/k/v of 3072 rows x 512 300 tokens
+// 12.3 / 10.1; 7 % over a grid of public calls.  It loses up to 6 % at some sizes
+// (2048 x 4096 600 tokens 32.0 / 33.8, 2048 x 2048 256 tokens 16.0 / 17.0).
+static float shape_us(uint32_t n_tok, uint32_t ct, uint32_t slabs, float outputs, const GemmShape &s, bool summed) {
+    // (a few ns per shape: every count is a power of two)
+    const bool small = s.bt == 64;
+    const float lone = small ? 0.8f : 1.14f, shared = (small ? 0.69f : 0.97f) * s.groups, start = small ? 0.1f : 0.9f;
+    const uint32_t g = s.groups >> 1, p = s.ksplit >> 1, cap = (small ? 2u : 1u) - g;     // logarithms
+    const uint32_t wgs = (ct * ((n_tok + s.bt - 1) >> (small ? 6 : 7))) << p, room = 8 + cap;
+    const uint32_t full = wgs >> room, rest = (wgs - (full << room) + 255) >> 8;
+    const float walk = (float)((slabs + (1u << (g + p)) - 1) >> (g + p));
+    auto round = [&](uint32_t per_cu) { return start + walk * fmaxf(shared * per_cu, lone); };
+    float us = full * round(1u << cap) + (rest ? round(rest) : 0.0f) + (g ? (small ? 0.5f : 1.75f) : 0.0f);
+    if (p) us += (summed ? 1.0f : 1.77f) * 1e-6f * outputs * s.ksplit + (summed ? 0.0f : 2.33f);
+    return us;
+}
+static GemmShape gemm_shape(uint32_t nmat, uint32_t n_tok, uint32_t ct, uint32_t K, uint32_t rows, uint32_t max_parts,
+                            bool summed) {
     const uint32_t T = ct * ((n_tok + 127) / 128), T4 = T / 2, slabs = (K + 127) / 128;
     if (K % 128 == 0 && T4 >= 448 && (T4 >= 2048 || T4 % 512 >= 448 || T4 % 512 == 0)) return {true, 128, 1, 1};
-    if (nmat == 2 || T >= 360) return {false, 128, 1, 1};
-    if (slabs < 4) return {false, T < 200 ? 64u : 128u, 1, 1};
-    if (max_parts >= 4 && slabs >= 64) return {false, 128, T < 60 ? 2u : 1u, 2 * T >= 360 ? 2u : 4u};
-    if (T >= 160) return {false, 128, 2, 1};
-    const uint32_t T64 = ct * ((n_tok + 63) / 64);
-    if (n_tok <= 256 || T <= 64) {
-        if (T64 >= 160 || slabs < 8 || max_parts < 2) return {false, 64, 1, 1};
-        return max_parts >= 4 && slabs >= 16 ? GemmShape{false, 64, 1, 4} : GemmShape{false, 64, 2, 2};
-    }
-    return {false, 128, 2, slabs < 8 || max_parts < 2 ? 1u : 2u};
+    GemmShape best{false, 128, 1, 1};
+    if (nmat == 2 || T >= 360) return best;
+    const float outputs = (float)n_tok * rows;
+    float least = 1e30f;
+    for (const uint32_t bt : {64u, 128u})
+        for (const uint32_t g : {1u, 2u})
+            for (uint32_t ks = 1; ks <= max_parts && ks * g <= slabs; ks *= 2) {
+                // (the public calls' parts lie in the context's scratch)
+                if (ks > 1 && !summed && (double)ks * n_tok * rows * 4 > (double)kGemmScratch) break;
+                const GemmShape s{false, bt, g, ks};
+                const float us = shape_us(n_tok, ct, slabs, outputs, s, summed);
+                if (us < least) {
+                    least = us;
+                    best = s;
+                }
+            }
+    return best;
 }
 
 template <int NMAT, bool REP>
@@ -451,12 +472,13 @@ static uint32_t gemm_cols(int nmat, int nseg, const uint32_t *M) {
 // is not split.
 static int gemm_run(chn_ctx *ctx, int nmat, int nseg, const float *X, const uint32_t *const *W, const uint32_t *W1,
                     float *const *Y, const uint32_t *M, uint32_t n_tok, uint32_t K, __bf16 *xb, bool repacked,
-                    __bf16 *Yb, PartialOut *po, float *scratch) {
+                    __bf16 *Yb, PartialOut *po, float *scratch, uint32_t yb_ntt = 0) {
     hipStream_t st = ctx->stream;
-    const uint32_t yb_ntt = Yb && !X ? xb_layout(n_tok, 1, M[0]) : 0;    // the down projection's order
+    uint32_t rows = 0;
+    for (int s = 0; s < nseg; ++s) rows += M[s];
     if (po) po->parts = 1;
     if (Yb && nmat == 1) return set_err(ctx, CHN_E_UNSUPPORTED, "bf16 output needs the two-matrix contraction");
-    if (few_tokens(n_tok, nmat, K)) {
+    if (few_tokens(n_tok, nmat, K, rows, nseg)) {
         if (X && launch_to_bf16_few(st, X, xb, n_tok, K)) return hip_fail(ctx, hipGetLastError(), "k_to_bf16_few");
         if (launch_q4gemm_few(st, nmat, nseg, W, W1, Y, M, n_tok, K, xb, repacked, Yb, yb_ntt))
             return hip_fail(ctx, hipGetLastError(), "k_q4gemm_few");
@@ -475,9 +497,7 @@ static int gemm_run(chn_ctx *ctx, int nmat, int nseg, const float *X, const uint
     a.n_tok = n_tok;
     a.K = K;
     const uint32_t max_parts = nseg > 1 ? 1 : (scratch ? 4 : (po ? po->max_parts : 1));
-    GemmShape sh = gemm_shape(nmat, n_tok, gemm_cols(nmat, nseg, M), K, max_parts);
-    // (fits by the rule: it splits less than 360 tiles of 64 KB in two, less than 180 in four)
-    if (scratch && (size_t)sh.ksplit * n_tok * M[0] * 4 > kGemmScratch) sh.ksplit = 1;
+    const GemmShape sh = gemm_shape(nmat, n_tok, gemm_cols(nmat, nseg, M), K, rows, max_parts, !scratch);
     if (sh.ksplit > 1 && scratch) {
         a.Y[0] = scratch;
         a.ypart = (size_t)n_tok * M[0];
@@ -505,8 +525,9 @@ static int gemm_run(chn_ctx *ctx, int nmat, int nseg, const float *X, const uint
 }
 
 int launch_q4gemm(chn_ctx *ctx, int nmat, const float *X, const uint32_t *W0, const uint32_t *W1, float *Y,
-                  uint32_t n_tok, uint32_t M, uint32_t K, __bf16 *xb, bool repacked, __bf16 *Yb, PartialOut *po) {
-    return gemm_run(ctx, nmat, 1, X, &W0, W1, &Y, &M, n_tok, K, xb, repacked, Yb, po, nullptr);
+                  uint32_t n_tok, uint32_t M, uint32_t K, __bf16 *xb, bool repacked, __bf16 *Yb, PartialOut *po,
+                  uint32_t yb_ntt) {
+    return gemm_run(ctx, nmat, 1, X, &W0, W1, &Y, &M, n_tok, K, xb, repacked, Yb, po, nullptr, yb_ntt);
 }
 
 // q, k and v of one layer in one launch: three repacked matrices over the
@@ -522,8 +543,9 @@ int launch_q4gemm_qkv(chn_ctx *ctx, const float *X, const uint32_t *Wq, const ui
 }
 
 // The public calls' buffer for the bf16 activations (kGemmScratch).
-static int public_activations(chn_ctx *ctx, uint32_t n_tok, int nmat, uint32_t K, __bf16 *&xb) {
-    if (few_tokens(n_tok, nmat, K)) {
+static int public_activations(chn_ctx *ctx, uint32_t n_tok, int nmat, uint32_t K, uint32_t rows, int nseg,
+                              __bf16 *&xb) {
+    if (few_tokens(n_tok, nmat, K, rows, nseg)) {
         xb = (__bf16 *)ctx->gemm_scratch;
         return CHN_OK;
     }
@@ -541,7 +563,7 @@ static int gemm_common(chn_ctx *ctx, int nmat, const uint32_t *W0, const uint32_
                 "weights must be %d-byte aligned", repacked ? 16 : 4);
     if (!n_tok || !M) return CHN_OK;
     __bf16 *xb = nullptr;
-    int rc = public_activations(ctx, n_tok, nmat, K, xb);
+    int rc = public_activations(ctx, n_tok, nmat, K, M, 1, xb);
     if (rc) return rc;
     return gemm_run(ctx, nmat, 1, X, &W0, W1, &Y, &M, n_tok, K, xb, repacked, Yb, nullptr, (float *)ctx->gemm_scratch);
 }
@@ -587,7 +609,7 @@ extern "C" int chn_batch_qkv_q4r(chn_ctx *ctx, const void *Wq, const void *Wk, c
     CHN_REQUIRE(ctx, aligned(X, 16) && aligned(Wq, 16) && aligned(Wk, 16) && aligned(Wv, 16), "misaligned argument");
     if (!n_tok || !q_dim || !kv_dim) return CHN_OK;
     __bf16 *xb = nullptr;
-    int rc = public_activations(ctx, n_tok, 1, K, xb);
+    int rc = public_activations(ctx, n_tok, 1, K, q_dim + 2 * kv_dim, 3, xb);
     if (rc) return rc;
     return launch_q4gemm_qkv(ctx, X, (const uint32_t *)Wq, (const uint32_t *)Wk, (const uint32_t *)Wv, Yq, Yk, Yv,
                              n_tok, q_dim, kv_dim, K, xb);

@@ -1,6 +1,6 @@
 // Batched contractions over Q4 weights for few tokens (a short message, the
 // tail of a prompt): gemm_q4.hip's contractions (shaders/batch_gemm_q4.wgsl,
-// shaders/batch_fused_mlp_q4.wgsl) for n_tok <= kFewTokens.
+// shaders/batch_fused_mlp_q4.wgsl) where few_tokens holds.
 //
 // What bounds them: reading the weights (gate/up at 12B dims: 66 MB against
 // 8.5 GFLOP at 24 tokens), then turning them into bf16 (21 VALU operations
@@ -256,18 +256,16 @@ static void launch_few_nt(hipStream_t st, FewArgs &a) {
 
 template <int NMAT, bool REP>
 static void launch_few_shape(hipStream_t st, FewArgs &a, int nseg) {
-    // 32 features per workgroup where that leaves about one workgroup per CU
     uint32_t rows = 0;
     for (int s = 0; s < nseg; ++s) rows += a.M[s];
-    const bool wide = rows / 32 >= 240;
-    const uint32_t per = wide ? 32 : 16;
+    const uint32_t per = few_features(rows);
     uint32_t g = 0;
     for (int s = 0; s < 3; ++s) {
         a.g0[s] = s < nseg ? g : 0xffffffffu;
         if (s < nseg) g += (a.M[s] + per - 1) / per;
     }
     a.ngrp = g;
-    if (wide) launch_few_nt<NMAT, 2, REP, 4>(st, a);
+    if (per == 32) launch_few_nt<NMAT, 2, REP, 4>(st, a);
     else launch_few_nt<NMAT, 1, REP, 8>(st, a);
 }
 

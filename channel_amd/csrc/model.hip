@@ -212,20 +212,12 @@ static int alloc_runtime(chn_model *m) {
     m->pfrag_bytes = prefill_frag_bytes(md.kvd / 256 ? md.kvd / 256 : 1, kSlotsMax + T);
     M_ALLOC(m->pfrag, m->pfrag_bytes);
     M_ALLOC(m->prope, (size_t)2 * T * kRopePairs * sizeof(float2));
-    // bf16 operands: width I in pact, H or a layer's qd in pxb.  Few-token prefills pad
-    // tokens to 16 and K to 256 (xb_elems); larger ones take n * K.
-    auto xb_bytes = [&](uint32_t K) {
-        size_t most = (size_t)T * K;
-        for (const int nmat : {1, 2})
-            for (const uint32_t n : {T, kFewTokensWide, kFewTokens})
-                if (n <= T && xb_elems(n, K, nmat) > most) most = xb_elems(n, K, nmat);
-        return 2 * most;
-    };
-    size_t xb_most = xb_bytes(H);
+    // bf16 operands, in either order: width I in pact, H or a layer's qd in pxb
+    size_t xb_most = xb_elems(T, H);
     for (const auto &l : m->L)
-        if (xb_bytes(l.qd) > xb_most) xb_most = xb_bytes(l.qd);
-    M_ALLOC(m->pact, xb_bytes(I));
-    M_ALLOC(m->pxb, xb_most);
+        if (xb_elems(T, l.qd) > xb_most) xb_most = xb_elems(T, l.qd);
+    M_ALLOC(m->pact, 2 * xb_elems(T, I));
+    M_ALLOC(m->pxb, 2 * xb_most);
     M_ALLOC(m->pslots, (size_t)(kSlotsMax + T) * 4);
     M_ALLOC(m->ptok, (size_t)T * 4);
     hipError_t e = hipHostMalloc((void **)&m->h_x, H * 4);
@@ -897,7 +889,8 @@ extern "C" int chn_prefill(chn_model *m, const uint32_t *tokens, uint32_t n, con
     // Both lie in the order the contractions of n tokens read (xb_at).
     __bf16 *xb = m->pxb;
     __bf16 *actb = (__bf16 *)m->pact;
-    const uint32_t ntt_qkv = xb_layout(n, 1, H), ntt_gu = xb_layout(n, 2, H);
+    auto ntt_qkv = [&](uint32_t i) { return xb_layout(n, 1, H, m->L[i].qd + 2 * m->L[i].kvd, 3); };
+    const uint32_t ntt_gu = xb_layout(n, 2, H, I), ntt_down = xb_layout(n, 1, I, H);
     // the prompt's rotation angles, once per kind (sliding / full layers)
     const HeadShape hs[2] = {head_shape(c, false), head_shape(c, true)};
     const float thetas[2] = {c.rope_theta, c.rope_theta_full};
@@ -908,7 +901,7 @@ extern "C" int chn_prefill(chn_model *m, const uint32_t *tokens, uint32_t n, con
         const float theta = l.full ? c.rope_theta_full : c.rope_theta;
         if (i == 0)
             P_(launch_rmsnorm_chain(s, m->px, nullptr, nullptr, l.in_norm, xb, nullptr, H, n, eps, 1.0f, false, 1, 0,
-                                      ntt_qkv));
+                                      ntt_qkv(0)));
         const uint32_t D = l.D, nkv = l.nkv, qd = l.qd, kvd = l.kvd, gqa = l.gqa;
         P_(launch_q4gemm_qkv(ctx, nullptr, l.Wq, l.Wk, l.Wv, m->pq, m->pk, m->pv, n, qd, kvd, H, xb));
         // sliding layers see the last 1024 slots (shaders/batch_causal_attn.wgsl:53)
@@ -921,19 +914,20 @@ extern "C" int chn_prefill(chn_model *m, const uint32_t *tokens, uint32_t n, con
                                  num_prev_slots, start_clock, n, nq, nkv, D, l.rot, (int)c.k_eq_v, theta, eps,
                                  ptab[l.full ? 1 : 0], fuse ? m->pfrag : nullptr, m->pfrag_bytes, win));
         P_(launch_prefill_attn(s, m->pq, l.kc, l.vc, m->pslots, n, num_prev_slots, nq, D, kvd, gqa, 1.0f, win,
-                               nullptr, xb, m->pattn_ws, m->pfrag, m->pfrag_bytes, fuse, xb_layout(n, 1, qd)));
+                               nullptr, xb, m->pattn_ws, m->pfrag, m->pfrag_bytes, fuse, xb_layout(n, 1, qd, H)));
         const size_t pstride = (size_t)m->max_tok * H;
         PartialOut po_o{pstride, 2};
         P_(launch_q4gemm(ctx, 1, nullptr, l.Wo, nullptr, m->pmlp, n, H, qd, xb, true, nullptr, &po_o));
         P_(launch_rmsnorm_chain(s, m->px, m->pmlp, l.has_post_attn ? l.post_attn : nullptr, l.pre_ffn, xb, nullptr,
                                 H, n, eps, 1.0f, true, po_o.parts, pstride, ntt_gu));
-        P_(launch_q4gemm(ctx, 2, nullptr, l.Wg, l.Wu, nullptr, n, I, H, xb, true, actb));
+        P_(launch_q4gemm(ctx, 2, nullptr, l.Wg, l.Wu, nullptr, n, I, H, xb, true, actb, nullptr, ntt_down));
         PartialOut po_d{pstride, 4};
         P_(launch_q4gemm(ctx, 1, nullptr, l.Wd, nullptr, m->pmlp, n, H, I, actb, true, nullptr, &po_d));
         const bool last = i + 1 == c.num_layers;
         const float *next_norm = last ? m->final_norm : m->L[i + 1].in_norm;
         P_(launch_rmsnorm_chain(s, m->px, m->pmlp, l.has_post_ffn ? l.post_ffn : nullptr, next_norm, xb,
-                                last ? m->pn : nullptr, H, n, eps, l.scalar, true, po_d.parts, pstride, ntt_qkv));
+                                last ? m->pn : nullptr, H, n, eps, l.scalar, true, po_d.parts, pstride,
+                                last ? 0u : ntt_qkv(i + 1)));
         if ((i + 1) % 4 == 0 || i + 1 == c.num_layers) {
             if (i + 1 == c.num_layers && (logits_out || topk_ids)) {
                 CHN_HIP(ctx, hipMemcpyAsync(m->normed, m->pn + (size_t)(n - 1) * H, H * 4, hipMemcpyDeviceToDevice, s));

@@ -1,7 +1,7 @@
-"""GPU parity of the few-token contractions (n_tok <= 128, k_q4gemm_few) at
+"""GPU parity of the few-token contractions (few_tokens, k_q4gemm_few) at
 the edges of their tiles: 16-token tiles and groups of 1..4 of them, 16- and
 32-feature workgroups, K steps of 256 that end inside a step, a half or a
-block.  Bar as for the other MFMA contractions: 1e-4 against the
+block, and the sizes above 128 tokens that they take.  Bar as for the other MFMA contractions: 1e-4 against the
 bf16-operand model (the same operand roundings, so only the order of the
 fp32 sums differs: K * 2^-24 <= 1e-3 of the terms' magnitudes at worst,
 ~sqrt(K) * 2^-24 ~ 1e-5 in practice)."""
@@ -35,6 +35,9 @@ def _matrix(ctx, rows, K, seed, repacked):
     (33, 7681, 384),     # 32-feature workgroups, one row past the last, half a step at the end
     (65, 48, 2304),      # five tiles in groups of three and two; nine steps over eight waves
     (128, 100, 4128),    # eight tiles, two groups of four
+    (129, 300, 512),     # nine tiles in three groups, the shortest K above 128 tokens
+    (512, 1024, 1024),   # eight groups of four, the most workgroups and the longest K there
+    (401, 1000, 992),    # 26 tiles in seven groups, ragged K
 ])
 def test_few_gemm_parity(ctx, n_tok, M, K, repacked):
     W, Wh = _matrix(ctx, M, K, 70 + M, repacked)

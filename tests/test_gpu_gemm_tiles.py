@@ -15,20 +15,27 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("repacked", [False, True])
 @pytest.mark.parametrize("n_tok,M,K", [
-    (129, 130, 32),        # 64-token tiles, one block of K
-    (200, 300, 1056),      # 64-token tiles with K split in two times two, ragged K
-    (150, 140, 2080),      # 64-token tiles with K split in four, ragged K
-    (65, 200, 8224),       # long K above the wide limit: two groups, K split in four
-    (257, 70, 416),        # few tiles: 64 tokens beyond 256 too
-    (260, 260, 1184),      # the same with K split
-    (300, 7000, 160),      # fewer than four slabs: 64-token tiles
-    (300, 2903, 544),      # 128-token tiles of two groups, one with a slab less, odd row length
-    (300, 2900, 1056),     # two groups and K split in two
-    (300, 7001, 544),      # two groups alone (165 tiles)
-    (385, 11520, 96),      # one group (360 tiles), one ragged slab
+    # 64-token tiles, one group of waves
+    (129, 130, 32),        # one block of K
+    (257, 70, 416),        # a tile of one token
+    (300, 7000, 160),
+    (129, 2903, 1568),     # K split in two, ragged K, odd row length
+    (200, 300, 1056),      # K split in four, ragged K
+    # 64-token tiles, two groups
+    (513, 200, 672),       # one with a slab less
+    (513, 200, 768),
+    (129, 2903, 1312),     # K split in two
+    (65, 200, 8224),       # K split in four
+    # 128-token tiles, one group
+    (385, 11520, 96),      # 360 tiles, one ragged slab
+    (65, 5000, 3104),      # K split in four
+    # 128-token tiles, two groups
+    (257, 7001, 1440),     # one with a slab less, odd row length
+    (65, 9000, 3936),      # K split in two
+    (65, 4500, 5664),      # K split in four
     (130, 57300, 128),     # 256-feature tiles (448 of them), one slab
     (130, 57300, 384),     # an odd and an even number of slabs: both DMA slots, the hand-over of the weights
-    (250, 57100, 512),     # (the last group of tokens and of features partly and wholly past the end)
+    (250, 57300, 512),     # (the last group of tokens and of features partly and wholly past the end)
 ])
 def test_gemm_launch_shapes(ctx, n_tok, M, K, repacked):
     W = synth_q4_dev(ctx, M, K, 60 + M)
@@ -50,7 +57,7 @@ def test_gemm_launch_shapes(ctx, n_tok, M, K, repacked):
 
 
 @pytest.mark.parametrize("repacked", [False, True])
-@pytest.mark.parametrize("n_tok,M,K", [(65, 200, 352), (130, 28610, 128), (130, 28610, 384), (245, 28600, 256)])
+@pytest.mark.parametrize("n_tok,M,K", [(65, 200, 352), (130, 28610, 128), (130, 28610, 384), (245, 28610, 256)])
 def test_gate_up_launch_shapes(ctx, n_tok, M, K, repacked):
     """64 and (448 tiles, K % 128 == 0) 128 features of each matrix per workgroup."""
     W, Wh = [], []
