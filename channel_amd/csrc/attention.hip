@@ -1224,9 +1224,13 @@ __global__ __launch_bounds__(256) void k_prefill_attn_d512(const float *__restri
 
 // Parts of the key list at head_dim 512: until there are 400 workgroups (a
 // step's exchange leaves a lone workgroup's matrix cores idle; 200 tokens
-// after 411 on 4 KV heads: 2 parts 76, 4 parts 81 us), and so that a part's
-// sums run over about 1024 keys at most (their rounding grows with the
-// length: over 1600 keys 3.1e-7 in one part, 3.0e-7 in the per-token kernel).
+// after 411 on 4 KV heads: 2 parts 76, 4 parts 81 us), and two or four where
+// the list has more than 1024 or 2048 keys, since the rounding of a part's sums
+// grows with its length.  With kPaParts parts at most, a part of the longest
+// list (4096 slots and 4096 new tokens) has 2048 keys.  Error against 64 bits,
+// one workgroup per token as before and now: 64 tokens after 411 keys 2.6e-7 /
+// 2.4e-7, 1024 after 4096 4.3e-7 / 3.2e-7, 256 after 7900 5.1e-7 / 3.5e-7 (flat
+// scores 4.5e-7 / 2.6e-7).
 static uint32_t pa5_parts(uint32_t n_tok, uint32_t n_keys, uint32_t gqa, uint32_t num_kv) {
     const uint32_t wgs = (n_tok * gqa + 15) / 16 * num_kv;
     uint32_t parts = 1;
@@ -1444,7 +1448,6 @@ struct QkvRope {
     const uint32_t *slots;                       // batch: token t's slot is slots[slot_offset + t], its clock start_clock + t
     uint32_t slot_offset, start_clock, num_q, num_kv, D, rot;
     float theta, eps;
-    const float2 *tab;                           // (cos, sin) per token and pair (launch_rope_tab_batch), or NULL
 };
 
 // RMSNorm * w, then RoPE on pairs (d, d + rot/2), suffix past rot copied, for
@@ -1487,16 +1490,12 @@ __global__ __launch_bounds__(256) void k_qkv_rope(QkvRope a) {
     const uint32_t clock = a.step ? a.step[0] : a.start_clock + t;
     const uint32_t slot = a.step ? a.step[1] : a.slots[a.slot_offset + t];
     if ((uint32_t)tid < half) {
-        if (a.tab) {
-            cs[tid] = a.tab[(size_t)t * half + tid];
-        } else {
-            const float fe = (2.0f * (float)tid) / (float)a.rot;
-            const float freq = 1.0f / powf(a.theta, fe);
-            const float ang = (float)clock * freq;
-            float sn, c;
-            sincosf(ang, &sn, &c);
-            cs[tid] = float2{c, sn};
-        }
+        const float fe = (2.0f * (float)tid) / (float)a.rot;
+        const float freq = 1.0f / powf(a.theta, fe);
+        const float ang = (float)clock * freq;
+        float sn, c;
+        sincosf(ang, &sn, &c);
+        cs[tid] = float2{c, sn};
     }
     __syncthreads();
 #pragma unroll
@@ -1567,7 +1566,7 @@ int launch_qkv_rope(hipStream_t st, const float *q_in, const float *k_in, const 
                     const float *kw, float *q_out, float *kc, float *vc, const uint32_t *step, uint32_t num_q,
                     uint32_t num_kv, uint32_t D, uint32_t rot, int k_eq_v, float theta, float eps) {
     return launch_rope_any(st, QkvRope{q_in, k_in, k_eq_v ? k_in : v_in, qw, kw, q_out, kc, vc, step, nullptr, 0, 0,
-                                       num_q, num_kv, D, rot, theta, eps, nullptr}, 1);
+                                       num_q, num_kv, D, rot, theta, eps}, 1);
 }
 
 // Four heads per workgroup, one per wave, for D a multiple of 256 and the
@@ -1835,7 +1834,7 @@ int launch_batch_qkv_rope(hipStream_t st, const float *q_in, const float *k_in, 
         return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
     }
     return launch_rope_any(st, QkvRope{q_in, k_in, k_eq_v ? k_in : v_in, qw, kw, q_out, kc, vc, nullptr, slots,
-                                       slot_offset, start_clock, num_q, num_kv, D, rot, theta, eps, tab}, n_tok);
+                                       slot_offset, start_clock, num_q, num_kv, D, rot, theta, eps}, n_tok);
 }
 
 // (cos, sin) of (start_clock + t) * theta^(-2d / rot) for t < n_tok, d <

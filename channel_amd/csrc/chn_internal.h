@@ -318,13 +318,13 @@ __host__ __device__ inline size_t xb_at(uint32_t ntt, uint32_t width, uint32_t t
     const uint32_t half = (k >> 8) * 2 + ((k >> 5) & 1), g = (k >> 6) & 3, j = (k >> 3) & 3;
     return ((((size_t)half * ntt + (t >> 4)) * 4 + j) * 64 + g * 16 + (t & 15)) * 8 + (k & 7);
 }
-int launch_to_bf16_few(hipStream_t st, const float *X, __bf16 *xb, uint32_t n_tok, uint32_t K);
+void launch_to_bf16_few(hipStream_t st, const float *X, __bf16 *xb, uint32_t n_tok, uint32_t K);
 // nseg matrices over the same activations (nmat 1), or gate W[0] and up W1
 // (nmat 2).  Yb (nmat 2): the result as bf16 instead of Y[0], in xb_at order
 // for yb_ntt.
-int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1, float *const *Y,
-                      const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked,
-                      __bf16 *Yb = nullptr, uint32_t yb_ntt = 0);
+void launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1,
+                       float *const *Y, const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked,
+                       __bf16 *Yb = nullptr, uint32_t yb_ntt = 0);
 // W0/W1 in the reference Q4 layout, or in Q4R with repacked.  X (fp32) is
 // converted into xb (xb_elems); with X == NULL, xb already holds the bf16
 // activations, in xb_at order for xb_layout.

@@ -107,8 +107,8 @@ __device__ __forceinline__ void group_barrier(uint32_t *n, uint32_t target, int 
 //
 // Calls at 12B dims with their bf16 pass, before and now, us: 512 x 3840 ->
 // 15360 89 / 72; q/k/v 300 tokens 64 / 37, 512 tokens 51 / 43; gate/up 256
-// tokens 120 / 70, 512 tokens 126 / 124; down 512 tokens 97 / 84, 1024 tokens
-// 186 / 150; o_proj 512 tokens 38 / 32, 1024 tokens 69 / 46.
+// tokens 120 / 70, 512 tokens 126 / 124; down 512 tokens 98 / 81, 1024 tokens
+// 191 / 144; o_proj 512 tokens 40 / 33, 1024 tokens 74 / 47.
 //
 // RAG: K % 128 != 0, the last slab's missing blocks contribute exact zeros.
 template <int NMAT, int BT, int FT, int G, bool REP, bool RAG>
@@ -479,9 +479,12 @@ static int gemm_run(chn_ctx *ctx, int nmat, int nseg, const float *X, const uint
     if (po) po->parts = 1;
     if (Yb && nmat == 1) return set_err(ctx, CHN_E_UNSUPPORTED, "bf16 output needs the two-matrix contraction");
     if (few_tokens(n_tok, nmat, K, rows, nseg)) {
-        if (X && launch_to_bf16_few(st, X, xb, n_tok, K)) return hip_fail(ctx, hipGetLastError(), "k_to_bf16_few");
-        if (launch_q4gemm_few(st, nmat, nseg, W, W1, Y, M, n_tok, K, xb, repacked, Yb, yb_ntt))
-            return hip_fail(ctx, hipGetLastError(), "k_q4gemm_few");
+        if (X) {
+            launch_to_bf16_few(st, X, xb, n_tok, K);
+            CHN_LAUNCHED(ctx, "k_to_bf16_few");
+        }
+        launch_q4gemm_few(st, nmat, nseg, W, W1, Y, M, n_tok, K, xb, repacked, Yb, yb_ntt);
+        CHN_LAUNCHED(ctx, "k_q4gemm_few");
         return CHN_OK;
     }
     GemmArgs a{};

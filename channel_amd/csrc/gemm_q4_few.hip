@@ -4,11 +4,11 @@
 //
 // What bounds them: reading the weights (gate/up at 12B dims: 66 MB against
 // 8.5 GFLOP at 24 tokens), then turning them into bf16 (21 VALU operations
-// per 8 weights, ~8 us of the chip's VALU for gate/up).  The 128- and
-// 256-token tiles of gemm_q4.hip spend the same time on 8 tokens as on 256,
-// with one workgroup per CU walking all of K behind a barrier per 64.  Here
-// weights go from memory to registers in the order an MFMA operand holds
-// them, with no LDS and no barrier before the end:
+// per 8 weights, ~8 us of the chip's VALU for gate/up).  The 64- and 128-token
+// tiles of gemm_q4.hip take about as long for 8 tokens as for 128, each walking
+// its K behind a barrier per slab.  Here weights go from memory to registers in
+// the order an MFMA operand holds them, and activations too, with no LDS and no
+// barrier before the end:
 //  * v_mfma_f32_16x16x32_bf16 with the weights as A (16 features) and the
 //    tokens as B.  Lane (r, g) = (lane & 15, lane >> 4) loads whole 32-weight
 //    blocks of row r; word j of the block it holds is its A operand of one
@@ -35,10 +35,10 @@
 // per CU, else one tile and 8 waves: gate/up 15360 x 3840 at 24 tokens 26.0
 // against 31.1 us with one tile; down 3840 x 15360 17.6 against 24.8 us with
 // two.
-// Measured at 12B dims, weights from HBM, before (128-/256-token tiles) and
-// now, us: gate/up 8 tokens 111 / 23, 32 tokens 113 / 26, 64 tokens 118 / 38,
-// 128 tokens 118 / 77; down 55 / 14, 56 / 18, 57 / 26, 57 / 51; q/k/v 29 / 8,
-// 30 / 9, 31 / 12, 31 / 20; o_proj 18 / 6, 19 / 7, 19 / 9, 20 / 18.
+// Measured at 12B dims, weights from HBM, before (tiles of 128 or 256 tokens
+// that took weights through LDS) and now, us, 8 / 32 / 64 tokens: gate/up 111 ->
+// 23, 113 -> 26, 118 -> 38; down 55 -> 14, 56 -> 18, 57 -> 26; q/k/v 29 -> 8, 30 ->
+// 9, 31 -> 12 (128 tokens 31 -> 20); o_proj 18 -> 6, 19 -> 7, 19 -> 9.
 #include "chn_internal.h"
 
 namespace chn {
@@ -235,9 +235,8 @@ __global__ __launch_bounds__(256) void k_to_bf16_few(const float *__restrict__ x
     *(fbf16x2 *)(o + 2) = fbf16x2{(__bf16)v.z, (__bf16)v.w};
 }
 
-int launch_to_bf16_few(hipStream_t st, const float *X, __bf16 *xb, uint32_t n_tok, uint32_t K) {
+void launch_to_bf16_few(hipStream_t st, const float *X, __bf16 *xb, uint32_t n_tok, uint32_t K) {
     k_to_bf16_few<<<dim3((K / 4 + 255) / 256, n_tok), 256, 0, st>>>(X, xb, n_tok, K, xb_tiles(n_tok));
-    return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
 }
 
 template <int NMAT, int FT, bool REP, int WK>
@@ -269,9 +268,9 @@ static void launch_few_shape(hipStream_t st, FewArgs &a, int nseg) {
     else launch_few_nt<NMAT, 1, REP, 8>(st, a);
 }
 
-int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1, float *const *Y,
-                      const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked, __bf16 *Yb,
-                      uint32_t yb_ntt) {
+void launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const *W, const uint32_t *W1,
+                       float *const *Y, const uint32_t *M, uint32_t n_tok, uint32_t K, const __bf16 *xb, bool repacked,
+                       __bf16 *Yb, uint32_t yb_ntt) {
     FewArgs a{};
     a.X = xb;
     for (int s = 0; s < nseg; ++s) {
@@ -292,7 +291,6 @@ int launch_q4gemm_few(hipStream_t st, int nmat, int nseg, const uint32_t *const 
         if (repacked) launch_few_shape<1, true>(st, a, nseg);
         else launch_few_shape<1, false>(st, a, nseg);
     }
-    return hipGetLastError() == hipSuccess ? CHN_OK : CHN_E_HIP;
 }
 
 }  // namespace chn

@@ -34,12 +34,13 @@ def _cache(nslot, kvd, seed):
     (8, 2, 9, 120, 33),        # a window that starts inside a step, two tiles
     (2, 1, 40, 1000, 0),       # parts of a long list
     (8, 4, 3, 2200, 0),        # more than 2048 keys: four parts
+    (4, 4, 9, 5200, 0),        # parts of more than 1024 keys
     (16, 2, 260, 0, 0),        # enough workgroups for one part
     (4, 4, 70, 300, 100),      # parts whose first chunks a late query does not see
 ])
 def test_prefill_attn_512(ctx, nq, gqa, n, prev, window):
     kvd = nq // gqa * 512
-    kc, vc, perm = _cache(2304, kvd, n + prev)
+    kc, vc, perm = _cache(max(2304, prev + n), kvd, n + prev)
     slots = perm[: prev + n]
     q, got = _run(ctx, nq, gqa, n, prev, window, kc, vc, slots)
     want = oracle.batch_causal_attn(q, kc, vc, slots, n, prev, nq, 512, kvd, gqa, 1.0, window, oracle.NTHREADS)

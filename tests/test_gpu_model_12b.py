@@ -4,7 +4,7 @@ sliding window 512, theta 1e4 (sliding) / 1e6 (full).
 
 * Two layers (one sliding, one full) of the seeded synthetic model: a
   512-token prefill (the benchmark's prompt, so the prefill GEMMs take the
-  same tile shapes: q/k/v in one launch on 128 x 128 tiles, down split in
+  same tile shapes: q/k/v in one launch on 128-token tiles, down split in
   K, gate/up writing bf16) against the oracle's bf16-operand model
   (normwise 1e-2 on logits, every K/V row and the last normed row), then
   four decode steps through chn_decode_token against the oracle in fp32
@@ -115,9 +115,8 @@ def test_12b_layers_prefill_512_then_decode(two_layers):
 
 def test_12b_layers_prefill_ragged_tiles(two_layers):
     """A 300-token prefill at the 12B layer dims: every contraction's last
-    token tile is ragged (300 = 256 + 44 for the 256-token tiles of gate/up
-    and of down, whose K is split four ways; 2 x 128 + 44 for q/k/v and o)
-    and the attention's last query tile holds 44 of its 64 tokens; then a
+    token tile is ragged (300 = 2 x 128 + 44; K is split in two for o and
+    down) and the attention's last query tile holds 44 of its 64 tokens; then a
     second chunk of 212 tokens over those 300 slots.  Against the oracle's
     bf16-operand model as the 512-token test: logits, every K/V row of both
     layers and the last normed row; then a third chunk of 100 tokens after

@@ -15,15 +15,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n_tok,M,K,sample", [
-    (512, 15360, 3840, 12),    # config: prefill Q4 GEMM 512 x 3840 -> 15360 (128 x 128 tiles)
-    (300, 16400, 64, None),    # 128 x 128 tiles, ragged tokens and features, one K step
-    (512, 3840, 15360, 6),     # down_proj shape (128 x 128 tiles, K split in two)
-    (512, 2048, 3840, 6),      # k/v shape (128 x 64 tiles, K split in two)
-    (100, 200, 96, None),      # ragged: tokens, features and K not tile multiples
+    (512, 15360, 3840, 12),    # gate or up of a 512-token prompt: 128-token tiles, one group of waves
+    (300, 16400, 64, None),    # the same, ragged tokens and features, half a slab of K
+    (512, 3840, 15360, 6),     # down_proj: 128-token tiles of two groups, K split in two
+    (512, 2048, 3840, 6),      # k/v: 64-token tiles of two groups, K split in two
+    (100, 200, 96, None),      # few tokens: tokens, features and K not tile multiples
     (1, 130, 32, None),        # one token, one Q4 block
     (129, 64, 160, None),
-    # K % 64 == 0 takes the DMA-pipelined kernel: ragged tokens and features,
-    # and fewer K steps (1, 2, 3) than DMA groups in flight
+    # few tokens, 64-token tiles of one slab and a half, K split in four parts of a slab or less
     (100, 200, 128, None),
     (1, 70, 64, None),
     (257, 100, 192, None),
@@ -90,7 +89,7 @@ def _repacked(ctx, rows, K, seed):
 
 def test_batch_qkv_q4r_model_shape(ctx):
     """q, k and v at the 12B prefill shape in one launch of three segments
-    (512 x 3840 -> 4096 | 2048 | 2048, 128 x 128 tiles), every row."""
+    (512 x 3840 -> 4096 | 2048 | 2048, 128-token tiles of two groups), every row."""
     n_tok, K, qd, kvd = 512, 3840, 4096, 2048
     Rq, Wq = _repacked(ctx, qd, K, 31)
     Rk, Wk = _repacked(ctx, kvd, K, 32)
@@ -109,9 +108,9 @@ def test_batch_qkv_q4r_model_shape(ctx):
 
 
 @pytest.mark.parametrize("n_tok,M,K", [
-    (512, 3840, 4096),      # o_proj: 128 x 64 tiles
-    (512, 3840, 15360),     # down_proj: 128 x 128 tiles, K split in two
-    (200, 3840, 15360),     # down at a short prompt: 128 x 64 tiles, K split in two
+    (512, 3840, 4096),      # o_proj: 64-token tiles of two groups
+    (512, 3840, 15360),     # down_proj: 128-token tiles of two groups, K split in two
+    (200, 3840, 15360),     # down at a short prompt: the same, K split in four
 ])
 def test_batch_gemm_q4r_model_shapes(ctx, n_tok, M, K):
     R, Wh = _repacked(ctx, M, K, 40 + K)
