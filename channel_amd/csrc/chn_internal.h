@@ -272,14 +272,14 @@ int launch_quantize(hipStream_t st, int q8, const uint16_t *src, uint32_t *dst, 
 //  * two matrices or long K: gate/up at 12B dims 48 tokens 38 / 44, 64 tokens
 //    43 / 44, 80 tokens 51 / 46; down 48 tokens 31 / 40, 65 tokens 50 / 40;
 //  * else what counts is the rounds of workgroups (a CU holds one or two of
-//    them): up to 128 tokens 3840 x 4096 (480 of them) 80 tokens 17.7 / 19.9,
-//    100 tokens 21.6 / 18.6, 2048 x 4096 (256) 100 tokens 17.0 / 20.7, 5120 x
-//    2048 (640) 100 tokens 20.3 / 16.9, q/k/v of 8192 rows (512) 128 tokens
-//    21.0 / 26.8, of 10240 (640) 100 tokens 17.6 / 12.2;
+//    them): up to 128 tokens 3840 x 4096 (480 of them) 80 tokens 17.7 / 17.9,
+//    100 tokens 21.6 / 18.6, 2048 x 4096 (256) 100 tokens 13.8 / 16.8, 5120 x
+//    2048 (640) 100 tokens 20.3 / 16.9, q/k/v of 8192 rows x 3840 (512) 128
+//    tokens 27.8 / 27.4, of 10240 x 1024 (640) 100 tokens 18.1 / 12.6;
 //  * beyond, where K is so short that the larger kernels' third launch or
-//    empty CUs show: 1024 x 1024 129 tokens 6.8 / 11.3, 512 tokens 12.7 /
-//    13.5, 2048 x 1024 256 tokens 11.7 / 13.2; 1024 x 256 350 tokens 8.4 / 7.7,
-//    1536 x 2048 256 tokens 15.9 / 15.8.
+//    empty CUs show: 1024 x 1024 129 tokens 6.8 / 10.8, 512 tokens 12.7 /
+//    13.1, 2048 x 1024 256 tokens 11.6 / 13.0; but 1024 x 256 350 tokens 8.4 /
+//    7.7, 1536 x 2048 256 tokens 16.2 / 15.8.
 // kFewMaxK: 64 rows of it fit the contractions' scratch.
 constexpr uint32_t kFewMaxTokens = 512, kFewMaxK = 1u << 18;
 inline uint32_t xb_tiles(uint32_t n_tok) { return (n_tok + 15) / 16; }
